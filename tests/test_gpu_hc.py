@@ -308,3 +308,37 @@ def test_block_argument_errors(dev):
     # zero positions: nothing to do
     assert moe_block(d, site, nw, NORM_EPS, st[:0]).numel() == 0
     d.close()
+
+
+# Both forms of the projection kernel (384 positions and up take the second), at sizes that
+# are no multiple of its row tiles (16, 32), of its chunks' groups (256 and 1024 elements of
+# N * D) or of the finalize's vectors, and either side of the switch.
+@pytest.mark.parametrize("P,N,D", [(383, 4, 1040), (384, 4, 1040), (417, 3, 320), (385, 1, 64), (400, 2, 2080),
+                                   (399, 8, 136), (388, 5, 192), (17, 4, 4112), (1, 8, 8192), (387, 4, 8192)])
+def test_hc_prepare_many_positions(oracle, dev, P, N, D):
+    fn, base, scale = make_site(3 * P + N, N, D)
+    st = streams_of(P + D, P, N, D)
+    site = DeviceHcSite.from_numpy(fn, base, scale, N, 20, EPS, dev)
+    d = dev_f16(st, dev)
+    out, post, comb = hc_prepare(d, site, None)
+    rows = sorted({0, 1, 15, 16, 31, 32, P // 2, P - 2, P - 1} & set(range(P)))
+    coll, opost, ocomb = oracle.hc_prepare(np.ascontiguousarray(st[rows]), N, D, fn, base, scale, 20, EPS)
+    # the bounds of test_hc_prepare_vs_oracle
+    assert np.max(np.abs(post.cpu().numpy()[rows] - opost)) <= 2e-5
+    assert np.max(np.abs(comb.cpu().numpy()[rows] - ocomb)) <= 2e-5
+    check_f16(out[rows], coll, ulps=1, extra=collapse_cond(np.ascontiguousarray(st[rows])))
+    # a position's results are the same bits in a call of its own
+    for r in rows[:: max(1, len(rows) // 4)]:
+        one = hc_prepare(d[r:r + 1].contiguous(), site, None)
+        assert all(torch.equal(a[0], b[r]) for a, b in zip(one, (out, post, comb)))
+    nw = dev_f16(np.random.default_rng(D).normal(1.0, 0.2, size=D).astype(np.float16).view(np.uint16), dev)
+    assert torch.equal(hc_prepare(d, site, nw, NORM_EPS)[0], rms_norm(out, nw, NORM_EPS))
+
+
+@pytest.mark.parametrize("D", [2, 6, 130, 2046, 2050, 4094, 4098, 8190])
+def test_rms_norm_ragged_hidden(oracle, dev, D):
+    # rows that are no multiple of the kernel's 8-value vectors, either side of its vector
+    # counts; rows of 2 mod 4 values start 4-byte aligned
+    x = (np.random.default_rng(D).normal(size=(5, D))).astype(np.float16).view(np.uint16)
+    w = np.random.default_rng(D + 1).normal(1.0, 0.2, size=D).astype(np.float16).view(np.uint16)
+    check_f16(rms_norm(dev_f16(x, dev), dev_f16(w, dev), NORM_EPS), oracle.rms_norm(x, w, NORM_EPS), ulps=2)
