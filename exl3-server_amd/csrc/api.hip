@@ -2,6 +2,7 @@
 // Reference interface: src/trellis_gemm.h (muyouming/exl3-server).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cstring>
 #include <mutex>
@@ -78,6 +79,9 @@ LinearWs linear_ws(int in, int out, int64_t rows, int n) {
   return w;
 }
 
+// Calls of many rows (RowsPlan): the rotated rows (n, rows, in) f16 instead.
+size_t rows_ws(int in, int64_t rows, int n) { return align_up((size_t)n * rows * in * 2, 256); }
+
 exl3_status check_ws(void *ws, size_t bytes, size_t need) {
   if (need && (!ws || bytes < need))
     return fail(EXL3_ERR_WORKSPACE, "workspace too small: need " + std::to_string(need) +
@@ -100,6 +104,20 @@ exl3_status linear_core(const exl3_trellis_desc *members, int n, const uint16_t 
   if (rc) return rc;
   float *part = reinterpret_cast<float *>((char *)ws + lw.part_off);
   const int n_sl = qmv_slices(in);
+  // many rows: every weight decoded once per rb * 16 rows, over rows rotated beforehand into
+  // the workspace (reference-form weights, no explicit rows_per_pass, outputs and svh aligned
+  // for its paired loads and stores; a workspace that only holds the slice partials keeps
+  // the slice path: the bits are the same)
+  const exl3_tuning tn = tuning();
+  const bool reference = tn.weight_form == EXL3_FORM_REFERENCE || w0.codebook == EXL3_CB_MUL1;
+  RowsPlan plan{};
+  if (reference && tn.rows_per_pass <= 0) plan = rows_plan(in, out, rows, n < PtrTable::kMax ? n : PtrTable::kMax);
+  uintptr_t align = reinterpret_cast<uintptr_t>(y16) | reinterpret_cast<uintptr_t>(svh_stack) |
+                    (reinterpret_cast<uintptr_t>(y32) & 7 ? 1 : 0);
+  if (!svh_stack)
+    for (int i = 0; i < n; ++i) align |= reinterpret_cast<uintptr_t>(members[i].svh);
+  if (align & 3) plan.rb = 0;
+  if (plan.rb && ws_bytes < rows_ws(in, rows, n < PtrTable::kMax ? n : PtrTable::kMax)) plan.rb = 0;
   for (int c0 = 0; c0 < n; c0 += PtrTable::kMax) {
     const int cn = std::min(PtrTable::kMax, n - c0);
     PtrTable tr{}, su{}, sv{};
@@ -112,6 +130,15 @@ exl3_status linear_core(const exl3_trellis_desc *members, int n, const uint16_t 
     }
     const uint16_t *xc = x + (x_shared ? 0 : (int64_t)c0 * rows * in);
     const int64_t x_stride = x_shared ? 0 : rows * in;
+    if (plan.rb) {
+      uint16_t *xrot = reinterpret_cast<uint16_t *>(ws);
+      rc = launch_stage_rows(xc, x_stride, rows, in, cn, x_is_xhat ? nullptr : &su, xrot, st);
+      if (rc) return rc;
+      rc = launch_qmv_rows(w0, plan, tr, cn, xrot, rows, y32 ? y32 + (int64_t)c0 * rows * out : nullptr,
+                           y16 ? y16 + (int64_t)c0 * rows * out : nullptr, sv, st);
+      if (rc) return rc;
+      continue;
+    }
     // from x, the QMV kernel applies each member's input Hadamard while it stages rows
     rc = launch_qmv(w0, tr, cn, xc, x_stride, rows, part, st, x_is_xhat ? nullptr : &su);
     if (rc) return rc;
@@ -220,7 +247,10 @@ exl3_status exl3_trellis_hadamard(const uint16_t *x_f16, const float *x_f32, int
 size_t exl3_trellis_workspace_size(const exl3_trellis_desc *w, int64_t rows, int32_t n_members) {
   if (!w || rows < 0 || n_members <= 0) return 0;
   const int32_t chunk = n_members < PtrTable::kMax ? n_members : PtrTable::kMax;
-  return linear_ws(w->in_features, w->out_features, rows, chunk).total;
+  const size_t part = linear_ws(w->in_features, w->out_features, rows, chunk).total;
+  if (w->in_features <= 0 || w->out_features <= 0 || !rows_plan(w->in_features, w->out_features, rows, chunk).rb)
+    return part;
+  return std::max(part, rows_ws(w->in_features, rows, chunk));
 }
 
 exl3_status exl3_trellis_matmul_raw(const exl3_trellis_desc *w, const uint16_t *xhat,

@@ -73,6 +73,18 @@ exl3_status launch_qmv_finalize(int n, int n_sl, int64_t rows, int out, const fl
                                 float *y32, uint16_t *y16, const PtrTable &svh,
                                 hipStream_t st);
 
+// Calls of many rows (k_qmv_rows): 16-row blocks and waves per workgroup; rb = 0: the
+// slice-parallel k_qmv. xrot: (n, rows, in) f16, the rows rotated (with suh) in staged order.
+struct RowsPlan {
+  int rb, waves;
+};
+RowsPlan rows_plan(int in, int out, int64_t rows, int n);
+exl3_status launch_stage_rows(const uint16_t *x, int64_t x_member_stride, int64_t rows, int in, int n,
+                              const PtrTable *suh, uint16_t *xrot, hipStream_t st);
+exl3_status launch_qmv_rows(const exl3_trellis_desc &shape, const RowsPlan &p, const PtrTable &trellis, int n,
+                            const uint16_t *xrot, int64_t rows, float *y32, uint16_t *y16, const PtrTable &svh,
+                            hipStream_t st);
+
 // Hyper-connection prepare (csrc/hc.hip): site and shape checks, the partials' workspace,
 // and the two launches (projection partials, then finalize with the optional RMSNorm).
 exl3_status check_hc(const exl3_hc_site *hc, int D);

@@ -14,6 +14,7 @@
 #include "exl3_device.hpp"
 #include "exl3_internal.hpp"
 #include "qmv_core.hpp"
+#include "qmv_rows.hpp"
 
 using namespace exl3d;
 
@@ -224,6 +225,46 @@ __global__ __launch_bounds__(256) void k_qmv(exl3h::PtrTable trellis, int tiles_
   }
 }
 
+// The rows of calls that take k_qmv_rows: member m's input Hadamard of every row (suh) or,
+// rotate = 0, the rows as they are, in the staged k order (stage_pair). One wave per (member,
+// row, kStageBatch blocks of 128), their butterfly stages interleaved.
+constexpr int kStageBatch = 8;
+
+// Bound by memory: 1000 rows of 8192 are 33 MB in and out.
+__global__ __launch_bounds__(256) void k_stage_rows(const uint16_t *__restrict__ x, int64_t x_member_stride,
+                                                    int64_t rows, int in, int n, exl3h::PtrTable suh, int rotate,
+                                                    uint16_t *__restrict__ xrot) {
+  const int lane = threadIdx.x & 63, nblk = in / 128, per_row = (nblk + kStageBatch - 1) / kStageBatch;
+  const int64_t gw = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (gw >= (int64_t)n * rows * per_row) return;
+  const int b0 = (int)(gw % per_row) * kStageBatch;
+  const int64_t mr = gw / per_row, row = mr % rows;
+  const int member = (int)(mr / rows);
+  const uint16_t *xr = x + member * x_member_stride + row * in + 2 * lane;
+  const uint16_t *su = (const uint16_t *)suh.p[member] + 2 * lane;
+  uint32_t *out = reinterpret_cast<uint32_t *>(xrot + mr * in);
+  uint32_t hx[kStageBatch];
+#pragma unroll
+  for (int q = 0; q < kStageBatch; ++q) hx[q] = *reinterpret_cast<const uint32_t *>(xr + min(b0 + q, nblk - 1) * 128);
+  if (rotate) {
+    float v0[kStageBatch], v1[kStageBatch], s0[kStageBatch], s1[kStageBatch];
+#pragma unroll
+    for (int q = 0; q < kStageBatch; ++q) {
+      const uint32_t sx = *reinterpret_cast<const uint32_t *>(su + min(b0 + q, nblk - 1) * 128);
+      v0[q] = f16_to_f32((uint16_t)(hx[q] & 0xffffu));
+      v1[q] = f16_to_f32((uint16_t)(hx[q] >> 16));
+      s0[q] = f16_to_f32((uint16_t)(sx & 0xffffu));
+      s1[q] = f16_to_f32((uint16_t)(sx >> 16));
+    }
+    wave_had_pre_n<kStageBatch>(v0, v1, s0, s1);
+#pragma unroll
+    for (int q = 0; q < kStageBatch; ++q) hx[q] = pack_f16x2(v0[q], v1[q]);
+  }
+#pragma unroll
+  for (int q = 0; q < kStageBatch; ++q)
+    if (b0 + q < nblk) stage_pair<false>(out, b0 + q, lane, hx[q]);
+}
+
 // One wave per (member, row, 128-column block): slice partials summed in slice order,
 // then the raw f32 result or the output Hadamard.
 __global__ __launch_bounds__(256) void k_qmv_finalize(int n, int n_sl, int64_t rows, int out,
@@ -367,6 +408,70 @@ int qmv_pass_rows(int64_t rows) {
 }
 
 int qmv_slices(int in) { return n_slices(in / 16); }
+
+// The linear's path: the slice-parallel k_qmv (16 rows per decode, f32 slice partials through
+// memory, the rotation repeated by every column block) or k_qmv_rows (64 or 128 rows per
+// decode, the whole k range in one workgroup) in one of its three shapes, whichever is
+// estimated faster. The estimates, in us, follow measurements at K = 4 (mcg) over in 640 to
+// 12288, out 1024 to 24576 and 17 to 1024 rows: the slice path takes 4.0 per 16 rows and
+// 2^24 weights; a workgroup of k_qmv_rows takes 27 (64 x 128 outputs), 42 (128 x 128) or 79
+// (128 x 256) per 4096 of k while every CU has one, and 35, 46 or 65 when it is alone.
+// 4096 x 4096, slice path against the estimate's choice: 38 against 38 at 128 rows, 68
+// against 43 at 256, 258 against 60 at 1024; 4096 x 24576: 44 against 40 at 17 rows, 1586
+// against 241 at 1024; 8192 x 4096 at 1000 rows: 495 against 101. Calls of up to 16 rows (one
+// decode either way) keep the slice path. rb = 0: the slice path.
+RowsPlan rows_plan(int in, int out, int64_t rows, int n) {
+  RowsPlan best{};
+  // (calls past the slice path's grid limit are refused there)
+  if (rows <= 16 || (int64_t)n_slices(in / 16) * ((rows + 15) / 16) > 65535) return best;
+  const double k = in / 4096.0;
+  double t_best = 4.0 + 4.0 * (double)((rows + 15) / 16) * ((double)in * out * n / (1 << 24));
+  const struct {
+    int rb, waves;
+    double alone, full;
+  } shapes[] = {{4, 4, 35, 27}, {8, 4, 46, 42}, {8, 8, 65, 79}};
+  for (const auto &s : shapes) {
+    const int64_t tiles = (rows + 16 * s.rb - 1) / (16 * s.rb);
+    const int64_t wgs = tiles * ((out / 32 + s.waves - 1) / s.waves) * n;
+    if (wgs > 0x7fffffff) continue;
+    const double t = 8.0 + k * std::max(s.alone, s.full * (double)((wgs + 255) / 256));
+    if (t < t_best) {
+      t_best = t;
+      best = RowsPlan{s.rb, s.waves};
+    }
+  }
+  return best;
+}
+
+exl3_status launch_stage_rows(const uint16_t *x, int64_t x_member_stride, int64_t rows, int in, int n,
+                              const PtrTable *suh, uint16_t *xrot, hipStream_t st) {
+  const int64_t waves = (int64_t)n * rows * ((in / 128 + kStageBatch - 1) / kStageBatch);
+  k_stage_rows<<<(unsigned)((waves + 3) / 4), 256, 0, st>>>(x, x_member_stride, rows, in, n, suh ? *suh : PtrTable{},
+                                                            suh ? 1 : 0, xrot);
+  EXL3_LAUNCHED("k_stage_rows");
+  return EXL3_OK;
+}
+
+exl3_status launch_qmv_rows(const exl3_trellis_desc &shape, const RowsPlan &p, const PtrTable &trellis, int n,
+                            const uint16_t *xrot, int64_t rows, float *y32, uint16_t *y16, const PtrTable &svh,
+                            hipStream_t st) {
+  exl3d::RowsArgs a{};
+  a.xrot = xrot;
+  a.rows = rows;
+  a.in = shape.in_features;
+  a.out = shape.out_features;
+  a.row_tiles = (int)((rows + 16 * p.rb - 1) / (16 * p.rb));
+  a.col_groups = (a.out / 32 + p.waves - 1) / p.waves;
+  a.members = n;
+  a.y32 = y32;
+  a.y16 = y16;
+  a.trellis = trellis;
+  a.svh = svh;
+  if (shape.K <= 4) launch_qmv_rows_k14(shape.K, shape.codebook, p.rb, p.waves, a, st);
+  else launch_qmv_rows_k58(shape.K, shape.codebook, p.rb, p.waves, a, st);
+  EXL3_LAUNCHED("k_qmv_rows");
+  return EXL3_OK;
+}
 
 exl3_status launch_qmv(const exl3_trellis_desc &shape, const PtrTable &trellis, int n,
                        const uint16_t *xhat, int64_t x_member_stride, int64_t rows, float *part,

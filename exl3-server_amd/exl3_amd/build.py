@@ -37,6 +37,7 @@ CFLAGS = [
 # the expert kernels' instantiations are spread over moe_experts_k*.hip so that they compile
 # in parallel (the longest first)
 SOURCES = ["moe_experts_k78.hip", "moe_experts_k56.hip", "moe_experts_k34.hip", "moe_experts_k12.hip",
+           "qmv_rows_k58.hip", "qmv_rows_k14.hip",
            "trellis_kernels.hip", "moe_experts.hip", "moe.hip", "api.hip", "loader.hip", "hc.hip"]
 
 

@@ -120,7 +120,8 @@ typedef struct {
 } exl3_tuning;
 
 /* What a trellis linear at `rows` rows will do. Mirrors TrellisPathInfo
- * (trellis_gemm.h:154-162). passes = weight streams per call. */
+ * (trellis_gemm.h:154-162). passes = weight streams per call, counted in MFMA passes of
+ * rows_per_block rows (calls of many rows decode a weight once for several of them). */
 typedef struct {
   int32_t staged;
   int32_t rows_per_block;
@@ -203,7 +204,10 @@ exl3_status exl3_trellis_hadamard(const uint16_t *x_f16, const float *x_f32, int
                                   exl3_stream_t stream);
 
 /* Workspace bytes for exl3_trellis_matmul_raw / exl3_trellis_linear(_grouped) on
- * n_members members of w's shape at `rows` rows. */
+ * n_members members of w's shape at `rows` rows: the f32 slice partials, or the rotated
+ * rows of a call of many rows where those are larger. (A workspace of the partials'
+ * n_members * (k slices) * rows * out * 4 bytes alone is enough for any call; the bits are
+ * the same.) */
 size_t exl3_trellis_workspace_size(const exl3_trellis_desc *w, int64_t rows, int32_t n_members);
 
 /* yhat = xhat @ W_hat (f32, (rows, out)); xhat already rotated. Replaces
