@@ -30,6 +30,7 @@ exl3_status launch_moe_expert(int which, int K, int cb, int64_t runs, const MoeA
 int moe_slices(int in);
 exl3_status launch_moe_act(const MoeArgs &a, int shared_mode, int dense_blocks, hipStream_t st);
 exl3_status launch_moe_rotate(const MoeArgs &a, int64_t slot0, int64_t n_slots, hipStream_t st);
+exl3_status launch_shared_dense(MoeArgs a, hipStream_t st);
 }
 
 namespace {
@@ -822,8 +823,8 @@ __device__ __forceinline__ void down_out(float2 y, uint32_t sv, float &y0, float
 
 // kFold: a long-run call (one folded down partial per slot, a.fold). Its variant holds
 // few enough VGPRs for 7 waves per SIMD (the general one: 4), so that many more rows'
-// loads are in flight over a long call's many rows; the f16 shared expert's partials are
-// then loaded after the ranks.
+// loads are in flight over a long call's many rows; the f16 shared expert's output is then
+// one f16 value, loaded after the ranks.
 template <bool kFold>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kFold ? 7 : 1))) void k_moe_combine(MoeArgs a) {
   const int lane = threadIdx.x & 63;
@@ -935,20 +936,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kFold ? 7 :
     r0 += y0;
     r1 += y1;
   } else if (a.shared_kind == exl3m::kSharedDense) {
-    if (kFold) load_dsh();
-    // dense_slots_sum's order over the two outputs' kDenseSlots partials
-    const int S = dense_mfma_splits(a.SI);
-    const float v0[8] = {dsh[0].x, dsh[0].y, dsh[0].z, dsh[0].w, dsh[1].x, dsh[1].y, dsh[1].z, dsh[1].w};
-    const float v1[8] = {dsh[2].x, dsh[2].y, dsh[2].z, dsh[2].w, dsh[3].x, dsh[3].y, dsh[3].z, dsh[3].w};
-    float d0 = v0[0], d1 = v1[0];
+    if constexpr (kFold) {  // k_shared_gemm's output, summed and rounded
+      const uint32_t v = *reinterpret_cast<const uint32_t *>(a.dsh_dn16 + (int64_t)row * a.H + c);
+      r0 += lo16(v);
+      r1 += hi16(v);
+    } else {
+      // dense_slots_sum's order over the two outputs' kDenseSlots partials
+      const int S = dense_mfma_splits(a.SI);
+      const float v0[8] = {dsh[0].x, dsh[0].y, dsh[0].z, dsh[0].w, dsh[1].x, dsh[1].y, dsh[1].z, dsh[1].w};
+      const float v1[8] = {dsh[2].x, dsh[2].y, dsh[2].z, dsh[2].w, dsh[3].x, dsh[3].y, dsh[3].z, dsh[3].w};
+      float d0 = v0[0], d1 = v1[0];
 #pragma unroll
-    for (int q = 1; q < 8; ++q)
-      if (q < S) {
-        d0 += v0[q];
-        d1 += v1[q];
-      }
-    r0 += rf16(d0);
-    r1 += rf16(d1);
+      for (int q = 1; q < 8; ++q)
+        if (q < S) {
+          d0 += v0[q];
+          d1 += v1[q];
+        }
+      r0 += rf16(d0);
+      r1 += rf16(d1);
+    }
   }
   const uint32_t o = pack_f16x2(r0, r1);
   *reinterpret_cast<uint32_t *>(a.out + (int64_t)row * a.H + c) = o;
@@ -1213,6 +1219,7 @@ MoeArgs make_args(const exl3_moe_layer_s *L, const MoeLayout &m, int64_t N, cons
   a.dsh_gu = (float *)(ws + m.dsh_gu);
   a.dsh_act = (uint16_t *)(ws + m.dsh_act);
   a.dsh_dn = (float *)(ws + m.dsh_dn);
+  a.dsh_dn16 = (uint16_t *)(ws + m.dsh_dn);
   a.xrot = (uint16_t *)(ws + m.xrot);
   a.out = out;
   return a;
@@ -1828,6 +1835,9 @@ exl3_status moe_layer_run(exl3_moe_layer_t layer, const uint16_t *h, int64_t N, 
   }
   const int H = layer->H;
   const bool dense_sh = layer->shared == exl3m::kSharedDense;
+  // the f16 shared expert: as tasks inside the expert launches, or (long-run calls) as two
+  // matrix products
+  const bool dense_tasks = dense_sh && !a.fold;
   const bool trellis_sh = layer->shared == exl3m::kSharedTrellis;
   const int64_t units = a.fold ? m.max_passes : m.R;  // work units: runs or long-run passes
   // Long-run calls: a trellis shared expert (under one wave of the machine on its own)
@@ -1876,6 +1886,10 @@ exl3_status moe_layer_run(exl3_moe_layer_t layer, const uint16_t *h, int64_t N, 
     const hipError_t e = hipEventRecord(layer->ev[1], st);
     if (e != hipSuccess) return fail_joined(hip_check(e, "hipEventRecord"));
   }
+  if (dense_sh && a.fold) {
+    rc = launch_shared_dense(a, st);
+    if (rc) return fail_joined(rc);
+  }
   // L3: routed gate/up (+ the f16 shared expert's gate/up partials), after the input
   // rotation of the routed slots (and of a trellis shared expert's slots when it runs on
   // this stream)
@@ -1883,7 +1897,7 @@ exl3_status moe_layer_run(exl3_moe_layer_t layer, const uint16_t *h, int64_t N, 
     rc = launch_moe_rotate(a, 0, (int64_t)a.P + (trellis_sh && !side ? N : 0), st);
     if (rc) return fail_joined(rc);
   }
-  rc = launch_moe_expert(0, layer->gu_K, kernel_cb(layer->gu_cb, a.weight_form), units, a, 0, dense_sh, st);
+  rc = launch_moe_expert(0, layer->gu_K, kernel_cb(layer->gu_cb, a.weight_form), units, a, 0, dense_tasks, st);
   if (rc) return fail_joined(rc);
   if (timed) {
     const hipError_t e = hipEventRecord(layer->ev[2], st);
@@ -1891,9 +1905,9 @@ exl3_status moe_layer_run(exl3_moe_layer_t layer, const uint16_t *h, int64_t N, 
   }
   // L4: routed SwiGLU activations (+ the f16 shared expert's SwiGLU), L5: routed down
   // (+ the f16 shared expert's down partials)
-  rc = launch_moe_act(a, 0, dense_sh ? shared_swiglu_blocks(N, layer->SI) : 0, st);
+  rc = launch_moe_act(a, 0, dense_tasks ? shared_swiglu_blocks(N, layer->SI) : 0, st);
   if (rc) return fail_joined(rc);
-  rc = launch_moe_expert(1, layer->dn_K, kernel_cb(layer->dn_cb, a.weight_form), units, a, 0, dense_sh, st);
+  rc = launch_moe_expert(1, layer->dn_K, kernel_cb(layer->dn_cb, a.weight_form), units, a, 0, dense_tasks, st);
   if (rc) return fail_joined(rc);
   if (timed) {
     const hipError_t e = hipEventRecord(layer->ev[3], st);

@@ -17,6 +17,8 @@
 // A trellis shared expert runs the gate/up, act and down kernels on one extra "run"
 // that holds every token row (three more launches; in long-run calls on the layer's
 // second stream, forked after the dispatch and joined before L6).
+// In long-run calls the f16 shared expert is two tiled matrix products before L3
+// (moe_shared.hip) instead of workgroups of L3, L4 and L5.
 // Calls of 32 rows or more add k_moe_rotate before L3 (each slot's gate/up input
 // rotated once); calls of 65 rows or more take the long-run gate/up and down kernels
 // over the pass table, and calls of 256 rows or more the tiled router logits kernel.
@@ -112,6 +114,7 @@ struct MoeArgs {
   float *dsh_gu;       // (2, N, SI, 8): f16 shared gate/up k-split partials
   uint16_t *dsh_act;   // (N, SI): f16 shared expert SwiGLU output
   float *dsh_dn;       // (N, H, 8): f16 shared down k-split partials
+  uint16_t *dsh_dn16;  // long-run mode: (N, H) f16 output of the f16 shared expert (dsh_dn's memory)
   uint16_t *out;       // (N, H)
   // Optional hyper-connection mix behind the combine (g5_hc_mix): with hc_out set, the
   // combine also writes hc_out[row][n] = post[n] * out[row] + (comb^T @ residual)[n]

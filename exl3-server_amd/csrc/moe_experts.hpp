@@ -486,18 +486,13 @@ __device__ __forceinline__ int long_item(int b, int per_unit, int shared_mode, c
 }
 
 template <int K, int CB, int PD>
-__global__ __launch_bounds__(kLongThreads) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_moe_gate_up_long(MoeArgs a, int shared_mode, int dense_blocks) {
+__global__ __launch_bounds__(kLongThreads) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_moe_gate_up_long(MoeArgs a, int shared_mode, int) {
   extern __shared__ uint32_t smem[];
   constexpr int kWaves = kLongThreads / 64;
-  if ((int)blockIdx.x < dense_blocks) {
-    shared_gate_up_block(a.h, a.N, a.H, a.SI, a.sh_dense[0], a.sh_dense[1], a.dsh_gu, blockIdx.x,
-                         kWaves);
-    return;
-  }
   const int out = shared_mode ? a.SI : a.I;
   const int n_np = out / 32, n_cb = (n_np + kWaves - 1) / kWaves;
   const int k_tiles = a.H / 16, ss = slice_steps(k_tiles), n_sl = n_slices(k_tiles);
-  int b = long_item(blockIdx.x - dense_blocks, 2 * n_cb, shared_mode, a);
+  int b = long_item(blockIdx.x, 2 * n_cb, shared_mode, a);
   if (b < 0) return;
   const int cb = b % n_cb;
   b /= n_cb;
@@ -569,17 +564,13 @@ __global__ __launch_bounds__(kLongThreads) __attribute__((amdgpu_waves_per_eu(4,
 }
 
 template <int K, int CB, int PD>
-__global__ __launch_bounds__(kLongThreads) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_moe_down_long(MoeArgs a, int shared_mode, int dense_blocks) {
+__global__ __launch_bounds__(kLongThreads) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_moe_down_long(MoeArgs a, int shared_mode, int) {
   extern __shared__ uint32_t smem[];
   constexpr int kWaves = kLongThreads / 64;
-  if ((int)blockIdx.x < dense_blocks) {
-    shared_down_block(a.dsh_act, a.N, a.H, a.SI, a.sh_dense[2], a.dsh_dn, blockIdx.x, kWaves);
-    return;
-  }
   const int in = shared_mode ? a.SI : a.I;
   const int n_np = a.H / 32, n_cb = (n_np + kWaves - 1) / kWaves;
   const int k_tiles = in / 16, ss = slice_steps(k_tiles), n_sl = n_slices(k_tiles);
-  const int b = long_item(blockIdx.x - dense_blocks, n_cb, shared_mode, a);
+  const int b = long_item(blockIdx.x, n_cb, shared_mode, a);
   if (b < 0) return;
   const int cb = b % n_cb, u = b / n_cb;
   RunInfo ri;

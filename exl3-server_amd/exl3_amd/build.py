@@ -38,7 +38,7 @@ CFLAGS = [
 # in parallel (the longest first)
 SOURCES = ["moe_experts_k78.hip", "moe_experts_k56.hip", "moe_experts_k34.hip", "moe_experts_k12.hip",
            "qmv_rows_k58.hip", "qmv_rows_k14.hip",
-           "trellis_kernels.hip", "moe_experts.hip", "moe.hip", "api.hip", "loader.hip", "hc.hip"]
+           "trellis_kernels.hip", "moe_experts.hip", "moe_shared.hip", "moe.hip", "api.hip", "loader.hip", "hc.hip"]
 
 
 def _compile(src: str) -> str:
