@@ -214,7 +214,7 @@ exl3_status launch_moe_expert(int which, int K, int cb, int64_t runs, const MoeA
   const int in = which == 0 ? a.H : (shared_mode ? a.SI : a.I);
   const int out = which == 0 ? (shared_mode ? a.SI : a.I) : a.H;
   const int n_sl = n_slices(in / 16);
-  const int waves = a.fold ? kLongThreads / 64 : kGuThreads / 64;
+  const int waves = (a.fold ? long_threads(dup_cb(cb)) : kGuThreads) / 64;
   if ((a.fold ? long_lds(in, K, cb) : expert_lds(in, a.pass_rows, waves, K, cb)) > 128 * 1024)
     return fail(EXL3_ERR_UNSUPPORTED, "expert kernel LDS above 128 KB");
   const int items = which == 0 ? a.gu_items : a.dn_items;

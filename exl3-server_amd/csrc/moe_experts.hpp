@@ -47,6 +47,7 @@
 #include "moe_common.hpp"
 #include "moe_dense.hpp"
 #include "qmv_core.hpp"
+#include "rows_lds.hpp"
 
 using namespace exl3d;
 using exl3m::MoeArgs;
@@ -258,8 +259,8 @@ __global__ __launch_bounds__(kDnThreads) __attribute__((amdgpu_waves_per_eu(kDnW
   }
 }
 
-// Long runs (calls of 65 token rows or more): 8-wave workgroups, wave w owns n-pair
-// 8*cb + w, passes of up to kLongRows rows with up to kLongBlocks 16-row MFMA blocks
+// Long runs (calls of 65 token rows or more): workgroups of 4 waves (8 in the halves form),
+// wave w owns n-pair 4*cb + w, passes of up to kLongRows rows with up to kLongBlocks 16-row MFMA blocks
 // per decode (qmv_slice_rb over the pass's occupied blocks only), and every k slice of
 // the tensor in one workgroup: each block's accumulators run on from the first k step
 // to the last (the reference's staged path likewise sums in its own association, within
@@ -267,7 +268,10 @@ __global__ __launch_bounds__(kDnThreads) __attribute__((amdgpu_waves_per_eu(kDnW
 // per output goes to slice position 0.
 using exl3m::kLongBlocks;
 using exl3m::kLongRows;
-constexpr int kLongThreads = 512;
+// Threads per workgroup: 4 waves, 128 columns (8 waves share a halves-form workgroup's 66 KB of
+// staged rows; in the reference form 4 measured as fast as 8, and 2% faster at 100 rows).
+constexpr int long_threads(bool dup) { return dup ? 512 : 256; }
+constexpr int kStageThreads = long_threads(true);  // stage_part's (halves form)
 // Staging loads in flight per lane: a slice of 64 plain rows is 64 x 64 chunks, 8 per
 // thread (two rounds of 4); a 4-step part of duplicated rows (the halves form) 64 x 32,
 // 4 per thread (one round).
@@ -277,8 +281,8 @@ constexpr int kStageBatchDn = 4;
 // Stages one part of a pass's rows into LDS: rows [0, nr) of the source, row r at byte
 // r * row_bytes of `src` (a buffer resource that covers exactly those nr rows), their
 // 16-byte chunks [kbyte0 / 16, kbyte0 / 16 + q_row) into staged rows xs + r * xs_stride.
-// Thread t takes chunk t % q_row of rows t / q_row + j * (kLongThreads / q_row) (q_row a
-// power of two that divides kLongThreads), so that its source offset and LDS row only
+// Thread t takes chunk t % q_row of rows t / q_row + j * (kStageThreads / q_row) (q_row a
+// power of two that divides kStageThreads), so that its source offset and LDS row only
 // step by whole rows; kBatch loads are issued before the first LDS store. A load of a row
 // at or past nr falls outside the resource and reads zero (no address clamps).
 template <bool kDup, int kBatch>
@@ -291,7 +295,7 @@ __device__ __forceinline__ void stage_part(__amdgpu_buffer_rsrc_t src, uint32_t 
   asm volatile("" : "+v"(tid));
   const int cq = tid & (q_row - 1);
   const int r0 = tid >> q_lg;
-  const int rstep = kLongThreads >> q_lg;
+  const int rstep = kStageThreads >> q_lg;
   const uint32_t vstep = (uint32_t)rstep * row_bytes;
   uint32_t vo = (uint32_t)r0 * row_bytes + (uint32_t)cq * 16 + kbyte0;
   uint32_t *dst = xs + r0 * xs_stride;
@@ -324,134 +328,102 @@ __device__ __forceinline__ void with_blocks(int nr, F &&pass) {
   }
 }
 
-// Double-buffered staging for the reference form (plain rows, one f16 per k-element):
-// passes run in parts of up to kDbSteps wave steps, and part t + 1's rows are copied into
-// the other of two LDS buffers by the 16-byte direct-to-LDS buffer load (lane i's 16
-// bytes land at the row's LDS address + 16 i, no register holds them) while part t is
-// decoded: one barrier per part, and the ring-word stream runs over the whole k range
-// with no break at the part boundaries. The buffers are two objects, so that the
-// compiler, which tracks the copies, does not hold reads of one buffer back for the copy
-// into the other. Every step meets the same A operands and accumulators as in the
-// single-buffered form, in the same order.
-constexpr int kDbSteps = 4;
-constexpr int kDbRowWords = kStepTiles * kDbSteps * 8 + 4;  // a part row + 4 words (bank offset)
-constexpr int kDbBufWords = kLongRows * kDbRowWords;
-static_assert(kLongThreads == 512, "eight waves copy a part's rows, wave + 8i");
-typedef __attribute__((address_space(3))) void lds_void_t;
-// The two part buffers: LDS of the plain-form long-run kernels only, the kernels that
+// Reference-form weights: the pass's rows go to two LDS buffers in parts of 2 wave steps
+// (rows_lds.hpp), part t + 2's copies issued when part t has been read, and the ring-word
+// stream runs over the whole k range. Every wave issues the same copies in every part (rows
+// past nr read zero), so that the compiler knows how many are in flight and a step waits for
+// its own ring words only; with copies under a condition it waited for all of them at the
+// first step of each part.
+static_assert(kLongBlocks == 4, "four waves copy a part's 64 rows, two or four loads each");
+constexpr int kLongBufWords = kLongRows * 4 * kRowsChunks;
+// The two part buffers: LDS of the reference-form long-run kernels only, the kernels that
 // reference them.
-__shared__ __align__(16) uint32_t g_db_a[kDbBufWords];
-__shared__ __align__(16) uint32_t g_db_b[kDbBufWords];
+__shared__ __align__(16) uint32_t g_db_a[kLongBufWords];
+__shared__ __align__(16) uint32_t g_db_b[kLongBufWords];
 
-// This wave's rows of a part (rows wave + 8i below nr): 16-byte chunks [0, q_row) of each
-// row from byte kbyte0 of the row, into buf.
-__device__ __forceinline__ void db_issue(__amdgpu_buffer_rsrc_t src, uint32_t row_bytes, uint32_t kbyte0,
-                                         int q_row, int nr, uint32_t *buf) {
+// One pass of up to 16 * NRB rows (nr >= 1) over the whole k range into D (from zero): rows
+// from src (row r at byte r * row_bytes, in the staged k order; nothing past nr), ring words of
+// n-pair np from base (a workgroup's 4 n-pairs are 128 columns: no wave is without). Ends
+// with a barrier and no copy in flight, so the buffers are free afterwards.
+template <int K, int CB, int PD, int NRB>
+__device__ __forceinline__ void long_pass_db(const uint32_t *base, int k_tiles, int tiles_n, int np,
+                                             __amdgpu_buffer_rsrc_t src, uint32_t row_bytes, u32x4 *slot,
+                                             f32x4 (&D)[NRB][2], uint32_t *dbA, uint32_t *dbB) {
+  static_assert(!dup_cb(CB), "reference-form weights");
+  constexpr int kW = long_threads(false) / 64;
+  const int total = k_tiles / kStepTiles, n_parts = total / kRowsPart;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-#pragma unroll
-  for (int i = 0; i < kLongRows / 8; ++i) {
-    const int r = wave + 8 * i;
-    if (r < nr && lane < q_row)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (lds_void_t *)(buf + r * kDbRowWords), 16,
-                                               (uint32_t)r * row_bytes + kbyte0 + 16u * (uint32_t)lane, 0, 0, 0);
-  }
-}
-
-// One pass of up to 16 * NRB rows (nr >= 1) of a plain-form tensor over its whole k range
-// into D (from zero): rows from src (row r at byte r * row_bytes, in the staged k order),
-// ring words of n-pair np from base; active = this wave has an n-pair (idle waves copy
-// rows and meet the barriers). Ends with a barrier, so the buffers are free afterwards.
-template <int K, int CB, int PD, int NRB, int kPart>
-__device__ __forceinline__ void long_pass_db_parts(const uint32_t *base, int k_tiles, int tiles_n, int np,
-                                                   bool active, __amdgpu_buffer_rsrc_t src, uint32_t row_bytes,
-                                                   int nr, u32x4 *slot, f32x4 (&D)[NRB][2], uint32_t *dbA,
-                                                   uint32_t *dbB) {
-  static_assert(!dup_cb(CB), "plain rows only");
-  static_assert(kPart <= kDbSteps && kPart % PD == 0, "part steps");
-  constexpr int kTw = tile_words(false);
-  const int total = k_tiles / kStepTiles;                   // wave steps over the k range
-  const int n_parts = total / kPart;
-  constexpr int q_row = kPart * kStepTiles * kTw / 4;       // 16-byte chunks of a part row
-  constexpr uint32_t part_bytes = 16u * q_row;
-  // part 0's copies before the stream's first loads: the copies of a part are always
-  // older than the ring loads in flight when the part's wait comes (below)
-  db_issue(src, row_bytes, 0, q_row, nr, dbA);
-  SliceStream<K, PD> S;
-  if (active) S.start(base, k_tiles, tiles_n, 0, np);
-  const StepLane sl = step_lane();
-  const int lane = threadIdx.x & 63;
-  const int wbase = (sl.kt * 2 + sl.nt) * 8 * K;
-  // block r's A operands: staged row 16r + l % 16 (rows past nr hold stale values: their
-  // MFMA rows are never stored, and an MFMA row depends on its own A row only), so the
-  // blocks' offsets differ by constants that fold into the LDS reads
-  const int xo0 = (lane & 15) * kDbRowWords + sl.kt * kTw;
-  int xo[NRB];
-#pragma unroll
-  for (int r = 0; r < NRB; ++r) {
-    xo[r] = xo0 + 16 * r * kDbRowWords;
-    D[r][0] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    D[r][1] = D[r][0];
-  }
-  // Loads complete in issue order. When part t's wait comes, a wave that decodes has
-  // exactly PD steps of ring loads in flight (PD * (K > 4 ? 2 : 1) loads), all issued
-  // after its copies of part t (at the start of part t - 1, or before the stream began):
-  // waiting until no more than those are outstanding completes the copies; an idle wave
-  // waits for everything. After the barrier every wave's copies of part t are in LDS, and
-  // no wave reads the other buffer (part t - 1) any more.
-  constexpr int kInFlight = PD * (K > 4 ? 2 : 1);
-  static_assert(kInFlight < 16, "vmcnt field");
-  auto run_part = [&](int t, uint32_t *cur, uint32_t *nxt) {
-    if (active)
-      __builtin_amdgcn_s_waitcnt(0x0F70 | kInFlight);  // vmcnt(kInFlight), expcnt/lgkmcnt unchecked
-    else
-      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    // The workgroup barrier without __syncthreads' fences, which count the copies as LDS
-    // writes and wait for every load in flight (vmcnt(0)), the ring words of the next
-    // steps included. The copies are complete by the wait above; this wave's LDS reads of
-    // the previous part have all been consumed by its MFMAs; the empty asm statements
-    // keep the compiler from moving memory operations across the barrier.
-    asm volatile("" ::: "memory");
+  const uint32_t vo = rows_voff<kW>(row_bytes, wave);
+  auto issue = [&](int t, uint32_t *buf) {  // (past the last part: beyond src, zeros and no access)
+    rows_issue<NRB <= 2 ? 2 : 4, kW>(src, vo, row_bytes, t < n_parts ? (uint32_t)t * (16 * kRowsChunks) : kPastEnd,
+                                     wave, buf);
+    rows_fence();
+  };
+  // Waits until this wave's copies of the next part are in LDS (`left`: the ring loads issued
+  // after them; loads complete in issue order) and its reads of the last one are done.
+  auto meet = [&](auto left) {
+    rows_fence();
+    __builtin_amdgcn_s_waitcnt(0x0070 | decltype(left)::value);
+    rows_fence();
     __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (t + 1 < n_parts) db_issue(src, row_bytes, (uint32_t)(t + 1) * part_bytes, q_row, nr, nxt);
-    if (active) {
+    rows_fence();
+  };
+  issue(0, dbA);
+  constexpr int kLoads = K > 4 ? 2 : 1;  // ring loads per step
+  SliceStream<K, PD> S;
+  S.start(base, k_tiles, tiles_n, 0, np);
+  const StepLane sl = step_lane();
+  const int wbase = (sl.kt * 2 + sl.nt) * 8 * K;
+  // A operand (step s of the part, half jp) of this lane's row: chunk 8s + 2kt + jp. Rows past
+  // nr: their MFMA rows are never stored, and an MFMA row depends on its own A row only.
+  int xo[kRowsPart][2];
 #pragma unroll
-      for (int sb = 0; sb < kPart; sb += PD) {
+  for (int s = 0; s < kRowsPart; ++s)
 #pragma unroll
-        for (int b = 0; b < PD; ++b) {
-          uint32_t W[K + 1];
-          step_words<K>(slot, wbase, sl.m, S.L[b], W);
-          // past the last step: lane offsets beyond the tensor (zeros, no memory access),
-          // so that every step issues the same loads
-          const int nx = t * kPart + sb + b + PD;
-          const bool past = nx >= total;
-          step_load<K>(S.rsrc, past ? S.vo0 + kPastEnd : S.vo0, past ? S.vo1 + kPastEnd : S.vo1,
-                       past ? 0u : S.so0 + (uint32_t)nx * S.step_bytes, S.L[b]);
-          mfma_step_rb<K, CB, NRB>(W, cur + (sb + b) * (kStepTiles * kTw), xo, D);
-        }
+    for (int jp = 0; jp < 2; ++jp)
+      xo[s][jp] = (lane & 15) * (4 * kRowsChunks) + 4 * ((8 * s + 2 * sl.kt + jp) ^ (lane & 15));
+#pragma unroll
+  for (int r = 0; r < NRB; ++r) D[r][0] = D[r][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  meet(std::integral_constant<int, PD * kLoads>{});
+  issue(1, dbB);
+  // Part t in cur; P: t % 2 (the ring registers of its steps).
+  auto run_part = [&](int t, auto P, uint32_t *cur) {
+#pragma unroll
+    for (int s = 0; s < kRowsPart; ++s) {
+      StepLoads<K> &L = S.L[(kRowsPart * decltype(P)::value + s) % PD];
+      uint32_t W[K + 1], F[K + 1];
+      step_words<K>(slot, wbase, sl.m, L, W);
+      // (past the last step: that one again)
+      step_load<K>(S.rsrc, S.vo0, S.vo1, S.so0 + (uint32_t)min(t * kRowsPart + s + PD, total - 1) * S.step_bytes, L);
+      lane_funnels<K>(W, F);
+      const f16x8 B0 = b_packed<K, CB, 0>(W, F), B1 = b_packed<K, CB, 4>(W, F);
+#pragma unroll
+      for (int r = 0; r < NRB; ++r) {
+        const f16x8 A0 = lds_a(cur + xo[s][0] + r * (16 * 4 * kRowsChunks));
+        D[r][0] = mfma16(A0, B0, D[r][0]);
+        D[r][1] = mfma16(A0, B1, D[r][1]);
+      }
+      const f16x8 B2 = b_packed<K, CB, 16>(W, F), B3 = b_packed<K, CB, 20>(W, F);
+#pragma unroll
+      for (int r = 0; r < NRB; ++r) {
+        const f16x8 A1 = lds_a(cur + xo[s][1] + r * (16 * 4 * kRowsChunks));
+        D[r][0] = mfma16(A1, B2, D[r][0]);
+        D[r][1] = mfma16(A1, B3, D[r][1]);
       }
     }
+    // the copies of part t + 1 were issued before this part's ring loads
+    meet(std::integral_constant<int, kRowsPart * kLoads>{});
+    issue(t + 2, cur);
   };
-  for (int t = 0; t < n_parts; t += 2) {
-    run_part(t, dbA, dbB);
-    if (t + 1 < n_parts) run_part(t + 1, dbB, dbA);
+  using P0 = std::integral_constant<int, 0>;
+  using P1 = std::integral_constant<int, 1>;
+  int t = 0;
+  for (; t + 2 <= n_parts; t += 2) {
+    run_part(t, P0{}, dbA);
+    run_part(t + 1, P1{}, dbB);
   }
-  __syncthreads();
-}
-
-// Parts of 4 wave steps where they divide the k range, else of 2 (a tensor's k range is
-// a multiple of 128, 2 wave steps): a part's steps unrolled, so that the loads in flight
-// at each part's wait are known to the compiler as they are to the wait.
-template <int K, int CB, int PD, int NRB>
-__device__ __forceinline__ void long_pass_db(const uint32_t *base, int k_tiles, int tiles_n, int np, bool active,
-                                             __amdgpu_buffer_rsrc_t src, uint32_t row_bytes, int nr,
-                                             u32x4 *slot, f32x4 (&D)[NRB][2], uint32_t *dbA, uint32_t *dbB) {
-  if ((k_tiles / kStepTiles) % kDbSteps == 0)
-    long_pass_db_parts<K, CB, PD, NRB, kDbSteps>(base, k_tiles, tiles_n, np, active, src, row_bytes, nr, slot, D,
-                                                 dbA, dbB);
-  else
-    long_pass_db_parts<K, CB, PD, NRB, 2>(base, k_tiles, tiles_n, np, active, src, row_bytes, nr, slot, D, dbA,
-                                          dbB);
+  if (t < n_parts) run_part(t, P0{}, dbA);
+  __builtin_amdgcn_s_waitcnt(0x0F70);
 }
 
 // Work unit u of the long-run kernels: pass u of the dispatch's pass table, or (shared
@@ -486,9 +458,9 @@ __device__ __forceinline__ int long_item(int b, int per_unit, int shared_mode, c
 }
 
 template <int K, int CB, int PD>
-__global__ __launch_bounds__(kLongThreads) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_moe_gate_up_long(MoeArgs a, int shared_mode, int) {
+__global__ __launch_bounds__(long_threads(dup_cb(CB))) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_moe_gate_up_long(MoeArgs a, int shared_mode, int) {
   extern __shared__ uint32_t smem[];
-  constexpr int kWaves = kLongThreads / 64;
+  constexpr int kWaves = long_threads(dup_cb(CB)) / 64;
   const int out = shared_mode ? a.SI : a.I;
   const int n_np = out / 32, n_cb = (n_np + kWaves - 1) / kWaves;
   const int k_tiles = a.H / 16, ss = slice_steps(k_tiles), n_sl = n_slices(k_tiles);
@@ -504,7 +476,7 @@ __global__ __launch_bounds__(kLongThreads) __attribute__((amdgpu_waves_per_eu(4,
   // uniform across the wave: in a scalar register, so that branches on it are scalar
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int np = cb * kWaves + wave;
-  const bool active = np < n_np;  // idle waves still stage rows and meet the barriers
+  const bool active = np < n_np;  // (halves form) idle waves still stage rows and meet the barriers
   constexpr bool kDup = dup_cb(CB);
   const int part = long_part_steps(k_tiles, kDup), n_parts = ss / part;
   const int part_k = kStepTiles * part * 16;
@@ -526,7 +498,7 @@ __global__ __launch_bounds__(kLongThreads) __attribute__((amdgpu_waves_per_eu(4,
       constexpr int NRB = decltype(nrb)::value;
       f32x4 D[NRB][2];
       if constexpr (!kDup) {
-        long_pass_db<K, CB, PD, NRB>(base, k_tiles, out / 16, np, active, src, row_bytes, nr, slot, D, g_db_a,
+        long_pass_db<K, CB, PD, NRB>(base, k_tiles, out / 16, np, src, row_bytes, slot, D, g_db_a,
                                      g_db_b);
       } else
       for (int sl = 0; sl < n_sl; ++sl) {
@@ -564,9 +536,9 @@ __global__ __launch_bounds__(kLongThreads) __attribute__((amdgpu_waves_per_eu(4,
 }
 
 template <int K, int CB, int PD>
-__global__ __launch_bounds__(kLongThreads) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_moe_down_long(MoeArgs a, int shared_mode, int) {
+__global__ __launch_bounds__(long_threads(dup_cb(CB))) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_moe_down_long(MoeArgs a, int shared_mode, int) {
   extern __shared__ uint32_t smem[];
-  constexpr int kWaves = kLongThreads / 64;
+  constexpr int kWaves = long_threads(dup_cb(CB)) / 64;
   const int in = shared_mode ? a.SI : a.I;
   const int n_np = a.H / 32, n_cb = (n_np + kWaves - 1) / kWaves;
   const int k_tiles = in / 16, ss = slice_steps(k_tiles), n_sl = n_slices(k_tiles);
@@ -598,7 +570,7 @@ __global__ __launch_bounds__(kLongThreads) __attribute__((amdgpu_waves_per_eu(4,
       constexpr int NRB = decltype(nrb)::value;
       f32x4 D[NRB][2];
       if constexpr (!kDup) {
-        long_pass_db<K, CB, PD, NRB>(tb.tr[2], k_tiles, a.H / 16, np, active, src, row_bytes, nr, slot, D,
+        long_pass_db<K, CB, PD, NRB>(tb.tr[2], k_tiles, a.H / 16, np, src, row_bytes, slot, D,
                                      g_db_a, g_db_b);
       } else
       for (int sl = 0; sl < n_sl; ++sl) {
@@ -648,7 +620,7 @@ static size_t expert_lds(int in, int pass_rows, int waves, int K, int cb) {
 // static LDS), then one ring-word slot per wave.
 static size_t long_lds(int in, int K, int cb) {
   return (dup_cb(cb) ? (size_t)kLongRows * long_row_words(in / 16, true) * 4 : 0) +
-         (size_t)(kLongThreads / 64) * slot_chunks(K) * 16;
+         (size_t)(long_threads(dup_cb(cb)) / 64) * slot_chunks(K) * 16;
 }
 
 // Per kernel instantiation: the one-time LDS attribute, set under std::call_once so that
@@ -686,9 +658,9 @@ static exl3_status moe_go(int which, dim3 blocks, hipStream_t st, const MoeArgs 
     if constexpr (PD <= 2) {  // long-run kernels keep at most 2 steps in flight (VGPRs)
       const size_t lds = long_lds(in, K, CB);
       static KernelAttr set_gu, set_dn;
-      return which == 0 ? launch_kernel(k_moe_gate_up_long<K, CB, PD>, blocks, kLongThreads, lds, st,
+      return which == 0 ? launch_kernel(k_moe_gate_up_long<K, CB, PD>, blocks, long_threads(dup_cb(CB)), lds, st,
                                         a, shared_mode, dense_blocks, set_gu)
-                        : launch_kernel(k_moe_down_long<K, CB, PD>, blocks, kLongThreads, lds, st, a,
+                        : launch_kernel(k_moe_down_long<K, CB, PD>, blocks, long_threads(dup_cb(CB)), lds, st, a,
                                         shared_mode, dense_blocks, set_dn);
     } else {
       return fail(EXL3_ERR_INVALID, "long-run expert kernels take at most 2 steps in flight");

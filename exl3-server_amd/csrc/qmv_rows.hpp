@@ -18,17 +18,10 @@
 #include "exl3_device.hpp"
 #include "exl3_internal.hpp"
 #include "qmv_core.hpp"
+#include "rows_lds.hpp"
 
 namespace exl3d {
 
-// Rows are copied to LDS in parts of 2 wave steps (a slice is 2, 4 or 8), double-buffered:
-// 256 bytes per row, unpadded, the 16-byte chunk c of row r at position c ^ (r % 16). A lane
-// of the 16-byte direct-to-LDS load lands at the next 16 bytes, so one load takes 4 rows,
-// and the 16 rows of an A operand read 16 different chunk positions (no bank conflicts).
-constexpr int kRowsPart = 2;                                   // wave steps per part
-constexpr int kRowsChunks = kRowsPart * kStepTiles * 8 / 4;    // 16-byte chunks of a row's part
-static_assert(kRowsChunks == 16, "one chunk position per row of an A operand");
-typedef __attribute__((address_space(3))) void rows_lds_t;
 // One of the two part buffers (objects of their own, so that reads of one are not held back
 // for the copies into the other); at the end it holds the f32 sums of 8 RB rows x 128 columns.
 template <int RB>
@@ -44,26 +37,6 @@ struct RowsArgs {
   exl3h::PtrTable trellis, svh;
 };
 
-// This wave's share of a part's rows: instruction i copies rows 4i .. 4i + 3 (rows past the
-// resource are zeros, not skipped, so that every wave issues the same number and the compiler
-// can count them). vo: the lane's offset of instruction `wave` at the row's start
-// (rows_voff); the lane's chunk position is the same in all of a wave's instructions, whose
-// rows are 4 WAVES apart.
-template <int WAVES>
-__device__ __forceinline__ uint32_t rows_voff(uint32_t row_bytes, int wave) {
-  static_assert(WAVES % 4 == 0, "rows 16n apart keep their chunk positions");
-  const uint32_t lane = threadIdx.x & 63, r = 4 * wave + (lane >> 4);
-  return r * row_bytes + 16u * ((lane & 15) ^ (r & 15));
-}
-template <int RB, int WAVES>
-__device__ __forceinline__ void rows_issue(__amdgpu_buffer_rsrc_t src, uint32_t vo, uint32_t row_bytes,
-                                           uint32_t kbyte0, int wave, uint32_t *buf) {
-#pragma unroll
-  for (int j = 0; j < 4 * RB / WAVES; ++j)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (rows_lds_t *)(buf + (wave + j * WAVES) * (16 * kRowsChunks)), 16,
-                                             vo + (kbyte0 + j * (4 * WAVES) * row_bytes), 0, 0, 0);
-}
-
 // f(integral_constant<int, 0>) .. f(integral_constant<int, N - 1>)
 template <int... I, typename F>
 __device__ __forceinline__ void rows_each(std::integer_sequence<int, I...>, F &&f) {
@@ -73,11 +46,6 @@ __device__ __forceinline__ void rows_each(std::integer_sequence<int, I...>, F &&
 // Position of column c of row r in the f32 tile (128 words a row): the four row groups of an
 // accumulator land on different banks.
 __device__ __forceinline__ int rows_col(int r, int c) { return c ^ (((r >> 2) & 1) << 5) ^ (((r >> 3) & 1) << 3); }
-
-__device__ __forceinline__ void rows_fence() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-}
 
 template <int K, int CB, int RB, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(RB > 4 || K > 5 ? 2 : 3))) void k_qmv_rows(RowsArgs a) {
