@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <utility>
 
 #include "exl3_device.hpp"
 #include "exl3_internal.hpp"
@@ -51,58 +52,126 @@ __global__ __launch_bounds__(256) void k_decode(const uint32_t *__restrict__ tre
 }
 
 // ---------------------------------------------------------------------------------
-// reconstruct: one workgroup per 128x128 block. The block is decoded into LDS as f32,
-// then the left butterflies (across rows), the row scale, the right butterflies
-// (across columns), the column scale and one RNE -- the operation order of
-// exl3.cpp:156-197, element for element.
+// reconstruct: one workgroup of 4 waves per 128x128 block, the operation order of
+// exl3.cpp:156-197 element for element: the left butterflies (across rows), the row scale,
+// the right butterflies (across columns), the column scale and one RNE.
+//
+// Bound by VALU issue beside the memory floor (about 8,500 wave instructions per block; 4096 x
+// 4096 K4: 16 us of issue, 42 MB or 8.2 us at 5.1 TB/s). The rows' butterflies stay in
+// registers: a thread decodes 2 columns x 32 rows straight from its ring words, the stages of
+// 1 to 16 rows are its own, those of 32 and 64 rows exchange lanes 16 and 32 apart. The block
+// then goes through LDS 64 rows at a time (32 KB, so 4 workgroups share a CU) to a wave per
+// row for the column stages and whole-row stores. Measured at that shape: 20 us, where
+// 14 barriered passes over the block in 66 KB of LDS took 121.
 // ---------------------------------------------------------------------------------
-template <int CB>
-__global__ __launch_bounds__(256) void k_reconstruct(const uint32_t *__restrict__ trellis, int K,
-                                                     int tiles_n, int out,
-                                                     const uint16_t *__restrict__ suh,
-                                                     const uint16_t *__restrict__ svh,
-                                                     uint16_t *__restrict__ w) {
-  __shared__ float buf[128][129];
-  const int cbk = blockIdx.x, rbk = blockIdx.y, tid = threadIdx.x;
-  for (int idx = tid; idx < 64 * 256; idx += 256) {
-    const int t = idx >> 8, p = idx & 255;
-    const int tr = t >> 3, tc = t & 7;
-    const uint32_t *tile =
-        trellis + ((int64_t)(rbk * 8 + tr) * tiles_n + (cbk * 8 + tc)) * 8 * K;
-    const int e = tile_element(p);
-    buf[tr * 16 + (e >> 4)][tc * 16 + (e & 15)] = (float)decode_one<CB>(tile_state_rt(tile, K, p));
+// v[i] <- the butterfly of v[i] and the value of the lane D (16 or 32) away.
+template <int D, int N>
+__device__ __forceinline__ void lane_butterfly(float (&v)[N]) {
+  const float sgn = (threadIdx.x & D) ? -1.0f : 1.0f;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    // r0 = the lower lane's value, r1 = the upper lane's, in both lanes
+    const int x = __builtin_bit_cast(int, v[i]);
+    const auto r = D == 32 ? __builtin_amdgcn_permlane32_swap(x, x, false, false)
+                           : __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    v[i] = __builtin_fmaf(sgn, __builtin_bit_cast(float, (int)r[1]), __builtin_bit_cast(float, (int)r[0]));
   }
-  __syncthreads();
-  for (int len = 1; len < 128; len <<= 1) {
-    for (int idx = tid; idx < 64 * 128; idx += 256) {
-      const int q = idx >> 7, c = idx & 127;
-      const int j = (q / len) * 2 * len + (q % len);
-      const float a = buf[j][c], b = buf[j + len][c];
-      buf[j][c] = a + b;
-      buf[j + len][c] = a - b;
+}
+
+template <int K, int CB, int T>
+__device__ __forceinline__ void decode_column_pair(const uint32_t (&W)[K + 1], const uint32_t (&F)[K + 1],
+                                                   float (&v)[2][32], int j) {
+  // stream position T of the lane's 32: k-row 2 (T / 8) + {0, 1, 8, 9}[T % 4], column half T / 4 % 2
+  constexpr int row = 2 * (T / 8) + (T % 4 < 2 ? T % 4 : T % 4 + 6);
+  v[T / 4 % 2][16 * j + row] = (float)decode_one<CB>(lane_state<K, T>(W, F));
+}
+template <int K, int CB, int... T>
+__device__ __forceinline__ void decode_columns(const uint32_t (&W)[K + 1], const uint32_t (&F)[K + 1],
+                                               float (&v)[2][32], int j, std::integer_sequence<int, T...>) {
+  (decode_column_pair<K, CB, T>(W, F, v, j), ...);
+}
+
+template <int K, int CB>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_reconstruct(
+    const uint32_t *__restrict__ trellis, int tiles_n, int out, const uint16_t *__restrict__ suh,
+    const uint16_t *__restrict__ svh, uint16_t *__restrict__ w) {
+  __shared__ __align__(16) float buf[64 * 128];
+  const int cbk = blockIdx.x, rbk = blockIdx.y;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  // lane: columns m and m + 8 of tile column 2 wave + lane / 8 % 2, rows 32 q .. 32 q + 31
+  const int m = lane & 7, tc = 2 * wave + ((lane >> 3) & 1), q = lane >> 4;
+  uint32_t W[2][K + 1];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const uint32_t *tile = trellis + ((int64_t)(rbk * 8 + 2 * q + j) * tiles_n + cbk * 8 + tc) * 8 * K;
+    W[j][0] = tile[(m * K + 8 * K - 1) % (8 * K)];
+#pragma unroll
+    for (int i = 0; i < K; ++i) W[j][i + 1] = tile[m * K + i];
+  }
+  float v[2][32];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    uint32_t F[K + 1];
+    lane_funnels<K>(W[j], F);
+    decode_columns<K, CB>(W[j], F, v, j, std::make_integer_sequence<int, 32>{});
+  }
+#pragma unroll
+  for (int len = 1; len < 32; len <<= 1)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < 32; ++i)
+        if (!(i & len)) {
+          const float a = v[h][i], b = v[h][i + len];
+          v[h][i] = a + b;
+          v[h][i + len] = a - b;
+        }
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    lane_butterfly<16>(v[h]);
+    lane_butterfly<32>(v[h]);
+  }
+  const uint16_t *su = suh + rbk * 128 + 32 * q;
+#pragma unroll
+  for (int i = 0; i < 32; ++i) {
+    const float s = f16_to_f32(su[i]) * kHadScale;
+    v[0][i] = v[0][i] * s;
+    v[1][i] = v[1][i] * s;
+  }
+  const uint16_t *sv = svh + cbk * 128 + 2 * lane;
+  const float t0 = f16_to_f32(sv[0]) * kHadScale, t1 = f16_to_f32(sv[1]) * kHadScale;
+  // 64 rows at a time; column c of a row whose bit 5 is set at c ^ 32, so that the two row
+  // quarters that write together fall on different banks
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    if (p) __syncthreads();  // the first half has been read
+    if ((q >> 1) == p) {
+      float *b = buf + (q & 1) * 32 * 128 + ((tc * 16 + m) ^ ((q & 1) * 32));
+#pragma unroll
+      for (int i = 0; i < 32; ++i) {
+        b[i * 128] = v[0][i];
+        b[i * 128 + 8] = v[1][i];  // (the swizzle leaves bit 3 alone)
+      }
     }
     __syncthreads();
-  }
-  for (int idx = tid; idx < 128 * 128; idx += 256) {
-    const int i = idx >> 7, c = idx & 127;
-    const float s = f16_to_f32(suh[rbk * 128 + i]) * kHadScale;
-    buf[i][c] = buf[i][c] * s;
-  }
-  __syncthreads();
-  for (int len = 1; len < 128; len <<= 1) {
-    for (int idx = tid; idx < 128 * 64; idx += 256) {
-      const int i = idx >> 6, q = idx & 63;
-      const int j = (q / len) * 2 * len + (q % len);
-      const float a = buf[i][j], b = buf[i][j + len];
-      buf[i][j] = a + b;
-      buf[i][j + len] = a - b;
+    constexpr int kB = 8;  // rows per wave at a time
+#pragma unroll 1
+    for (int r0 = kB * wave; r0 < 64; r0 += 4 * kB) {
+      float x0[kB], x1[kB];
+#pragma unroll
+      for (int i = 0; i < kB; ++i) {
+        const float2 x = *reinterpret_cast<const float2 *>(buf + (r0 + i) * 128 + ((2 * lane) ^ (r0 & 32)));
+        x0[i] = x.x;
+        x1[i] = x.y;
+      }
+      wave_fwht128_n<kB>(x0, x1);
+      uint16_t *o = w + (int64_t)(rbk * 128 + 64 * p + r0) * out + cbk * 128 + 2 * lane;
+#pragma unroll
+      for (int i = 0; i < kB; ++i) {
+        const uint32_t y = pack_f16x2(x0[i] * t0, x1[i] * t1);
+        __builtin_memcpy(o + (int64_t)i * out, &y, 4);
+      }
     }
-    __syncthreads();
-  }
-  for (int idx = tid; idx < 128 * 128; idx += 256) {
-    const int i = idx >> 7, c = idx & 127;
-    const float s = f16_to_f32(svh[cbk * 128 + c]) * kHadScale;
-    w[(int64_t)(rbk * 128 + i) * out + cbk * 128 + c] = f32_to_f16(buf[i][c] * s);
   }
 }
 
@@ -329,20 +398,28 @@ exl3_status launch_decode(const exl3_trellis_desc &w, uint16_t *w_hat, hipStream
   return EXL3_OK;
 }
 
-exl3_status launch_reconstruct(const exl3_trellis_desc &w, uint16_t *w_out, hipStream_t st) {
-  const int tiles_n = w.out_features / 16;
-  dim3 grid(w.out_features / 128, w.in_features / 128);
+template <int K>
+static void reconstruct_cb(const exl3_trellis_desc &w, uint16_t *w_out, hipStream_t st) {
+  const dim3 grid(w.out_features / 128, w.in_features / 128);
   const uint32_t *t = (const uint32_t *)w.trellis;
+  const int tiles_n = w.out_features / 16, out = w.out_features;
   switch (w.codebook) {
-    case 0:
-      k_reconstruct<0><<<grid, 256, 0, st>>>(t, w.K, tiles_n, w.out_features, w.suh, w.svh, w_out);
-      break;
-    case 1:
-      k_reconstruct<1><<<grid, 256, 0, st>>>(t, w.K, tiles_n, w.out_features, w.suh, w.svh, w_out);
-      break;
-    default:
-      k_reconstruct<2><<<grid, 256, 0, st>>>(t, w.K, tiles_n, w.out_features, w.suh, w.svh, w_out);
-      break;
+    case 0: k_reconstruct<K, 0><<<grid, 256, 0, st>>>(t, tiles_n, out, w.suh, w.svh, w_out); break;
+    case 1: k_reconstruct<K, 1><<<grid, 256, 0, st>>>(t, tiles_n, out, w.suh, w.svh, w_out); break;
+    default: k_reconstruct<K, 2><<<grid, 256, 0, st>>>(t, tiles_n, out, w.suh, w.svh, w_out);
+  }
+}
+
+exl3_status launch_reconstruct(const exl3_trellis_desc &w, uint16_t *w_out, hipStream_t st) {
+  switch (w.K) {
+    case 1: reconstruct_cb<1>(w, w_out, st); break;
+    case 2: reconstruct_cb<2>(w, w_out, st); break;
+    case 3: reconstruct_cb<3>(w, w_out, st); break;
+    case 4: reconstruct_cb<4>(w, w_out, st); break;
+    case 5: reconstruct_cb<5>(w, w_out, st); break;
+    case 6: reconstruct_cb<6>(w, w_out, st); break;
+    case 7: reconstruct_cb<7>(w, w_out, st); break;
+    default: reconstruct_cb<8>(w, w_out, st);
   }
   EXL3_LAUNCHED("k_reconstruct");
   return EXL3_OK;
