@@ -206,16 +206,19 @@ __global__ __launch_bounds__(256) void k_hadamard(const uint16_t *__restrict__ x
 }
 
 // ---------------------------------------------------------------------------------
-// QMV: grid (out/128 column blocks x k-slices, row passes, members); 4 waves per
-// workgroup, wave w owns n-pair 4*cb + w of one k-slice. The workgroup stages its
-// slice of up to 16 xhat rows into LDS in the MFMA k order and writes the slice
-// partials part[member][slice][row][col].
+// QMV: grid (groups of column blocks, k-slices x row passes, members); 4 waves per
+// workgroup, wave w owns n-pair 4*cb + w of each 128-column block cb of its group. The
+// workgroup stages its slice of up to 16 xhat rows into LDS in the MFMA k order and writes
+// the slice partials part[member][slice][row][col].
 // ---------------------------------------------------------------------------------
-template <int K, int CB, int PD>
-__global__ __launch_bounds__(256) void k_qmv(exl3h::PtrTable trellis, int tiles_n, int in,
+// Bound by decode VALU, the rotation of the rows beside it: a workgroup rotates its slice of
+// every row whatever its columns, so a group of blocks (kGroup) rotates once for all of them
+// and keeps one ring-word stream over them (waves per SIMD as in the expert kernels).
+template <int K, int CB, int PD, bool kGroup>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kGroup ? (K <= 4 ? 7 : 6) : 1))) void k_qmv(exl3h::PtrTable trellis, int tiles_n, int in,
                                              int out, const uint16_t *__restrict__ xhat,
                                              int64_t x_member_stride, int64_t rows,
-                                             int pass_rows, float *__restrict__ part,
+                                             int pass_rows, int group, float *__restrict__ part,
                                              exl3h::PtrTable suh, int rotate) {
   constexpr bool kDup = dup_cb(CB);
   // one ring-word slot per wave, then the slice's staged rows (pass_rows of them: the
@@ -226,15 +229,19 @@ __global__ __launch_bounds__(256) void k_qmv(exl3h::PtrTable trellis, int tiles_
   uint32_t *xs = reinterpret_cast<uint32_t *>(qmv_smem + 4 * slot_chunks(K));
   const int k_tiles = in / 16, ss = slice_steps(k_tiles), n_sl = n_slices(k_tiles);
   const int slice_k = kStepTiles * ss * 16, xs_stride = staged_row_words(k_tiles, kDup);
-  // grid: x = 128-column block, y = row block * n_sl + k-slice, z = member (one row
+  // grid: x = group of column blocks, y = row block * n_sl + k-slice, z = member (one row
   // block, the decode case, needs no division)
-  const int cb = blockIdx.x;
+  const int cb = kGroup ? blockIdx.x * group : blockIdx.x;
   const int sl = (int)gridDim.y == n_sl ? (int)blockIdx.y : (int)blockIdx.y % n_sl;
   const int64_t r0 = (int64_t)((int)gridDim.y == n_sl ? 0 : (int)blockIdx.y / n_sl) * pass_rows;
   const int nr = (int)min<int64_t>(pass_rows, rows - r0);
   const int member = blockIdx.z;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
 
+  // (a group's first ring words are in flight while the rows are staged)
+  SliceStream<K, PD> S;
+  if constexpr (kGroup)
+    S.start((const uint32_t *)trellis.p[member], k_tiles, tiles_n, sl * kStepTiles * ss, cb * 4 + wave);
   if (rotate) {
     // x, not xhat: the input Hadamard of the slice's 128-blocks (member's suh), in the
     // workgroup, kBatch blocks per wave at a time with every load issued first
@@ -279,18 +286,27 @@ __global__ __launch_bounds__(256) void k_qmv(exl3h::PtrTable trellis, int tiles_
     }
   }
   __syncthreads();
-  f32x4 D0, D1;
-  qmv_slice<K, CB, PD>((const uint32_t *)trellis.p[member], k_tiles, tiles_n, sl * kStepTiles * ss,
-                       cb * 4 + wave, ss, xs + min(lane & 15, nr - 1) * xs_stride,
-                       slots + wave * slot_chunks(K), D0, D1);
   float *p = part + (((int64_t)member * n_sl + sl) * rows + r0) * out + cb * 128 + wave * 32;
+  const uint32_t *xrow = xs + min(lane & 15, nr - 1) * xs_stride;
+  u32x4 *slot = slots + wave * slot_chunks(K);
+  auto store = [=](int it, const f32x4 &D0, const f32x4 &D1) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = d_row(i);
-    if (r < nr) {
-      p[(int64_t)r * out + d_col(0)] = D0[i];
-      p[(int64_t)r * out + d_col(1)] = D1[i];
+    for (int i = 0; i < 4; ++i) {
+      const int r = d_row(i);
+      if (r < nr) {
+        float *o = p + (int64_t)r * out + it * 128;
+        o[d_col(0)] = D0[i];
+        o[d_col(1)] = D1[i];
+      }
     }
+  };
+  if constexpr (kGroup) {
+    qmv_slice_items<K, CB, PD>(S, ss, min(group, out / 128 - cb), xrow, slot, store);
+  } else {
+    f32x4 D0, D1;
+    qmv_slice<K, CB, PD>((const uint32_t *)trellis.p[member], k_tiles, tiles_n, sl * kStepTiles * ss, cb * 4 + wave,
+                         ss, xrow, slot, D0, D1);
+    store(0, D0, D1);
   }
 }
 
@@ -437,8 +453,8 @@ exl3_status launch_hadamard(const uint16_t *x16, const float *x32, int64_t rows,
 
 template <int K, int CB, int PD>
 static void qmv_go(dim3 grid, hipStream_t st, const PtrTable &tr, int tiles_n, int in, int out,
-                   const uint16_t *xhat, int64_t xs, int64_t rows, int pass_rows, float *part,
-                   const PtrTable *suh) {
+                   const uint16_t *xhat, int64_t xs, int64_t rows, int pass_rows, int group,
+                   float *part, const PtrTable *suh) {
   // the wave slots and pass_rows staged rows (at most 16 x 2 KB + 8 KB: under the 64 KB
   // that a launch gets without an attribute)
   static_assert((size_t)4 * slot_chunks(8) * 16 +
@@ -447,33 +463,34 @@ static void qmv_go(dim3 grid, hipStream_t st, const PtrTable &tr, int tiles_n, i
                 "k_qmv LDS");
   const size_t lds = (size_t)4 * slot_chunks(K) * 16 +
                      (size_t)pass_rows * staged_row_words(in / 16, dup_cb(CB)) * 4;
-  k_qmv<K, CB, PD><<<grid, 256, lds, st>>>(tr, tiles_n, in, out, xhat, xs, rows, pass_rows, part,
-                                           suh ? *suh : PtrTable{}, suh ? 1 : 0);
+  const auto k = group > 1 ? k_qmv<K, CB, PD, true> : k_qmv<K, CB, PD, false>;
+  k<<<grid, 256, lds, st>>>(tr, tiles_n, in, out, xhat, xs, rows, pass_rows, group, part, suh ? *suh : PtrTable{},
+                            suh ? 1 : 0);
 }
 
 template <int K, int CB>
 static void qmv_pd(int pd, dim3 grid, hipStream_t st, const PtrTable &tr, int tiles_n, int in,
-                   int out, const uint16_t *xhat, int64_t xs, int64_t rows, int pass_rows,
+                   int out, const uint16_t *xhat, int64_t xs, int64_t rows, int pass_rows, int group,
                    float *part, const PtrTable *suh) {
   if (pd == 1)
-    return qmv_go<K, CB, 1>(grid, st, tr, tiles_n, in, out, xhat, xs, rows, pass_rows, part, suh);
+    return qmv_go<K, CB, 1>(grid, st, tr, tiles_n, in, out, xhat, xs, rows, pass_rows, group, part, suh);
   if constexpr (K <= 4) {
     if (pd >= 4)
-      return qmv_go<K, CB, 4>(grid, st, tr, tiles_n, in, out, xhat, xs, rows, pass_rows, part, suh);
+      return qmv_go<K, CB, 4>(grid, st, tr, tiles_n, in, out, xhat, xs, rows, pass_rows, group, part, suh);
   }
-  qmv_go<K, CB, 2>(grid, st, tr, tiles_n, in, out, xhat, xs, rows, pass_rows, part, suh);
+  qmv_go<K, CB, 2>(grid, st, tr, tiles_n, in, out, xhat, xs, rows, pass_rows, group, part, suh);
 }
 
 template <int K>
 static void qmv_cb(int cb, int pd, dim3 grid, hipStream_t st, const PtrTable &tr, int tiles_n,
-                   int in, int out, const uint16_t *xhat, int64_t xs, int64_t rows, int pass_rows,
+                   int in, int out, const uint16_t *xhat, int64_t xs, int64_t rows, int pass_rows, int group,
                    float *part, const PtrTable *suh) {
   switch (cb) {
-    case 0: qmv_pd<K, 0>(pd, grid, st, tr, tiles_n, in, out, xhat, xs, rows, pass_rows, part, suh); break;
-    case 1: qmv_pd<K, 1>(pd, grid, st, tr, tiles_n, in, out, xhat, xs, rows, pass_rows, part, suh); break;
-    case 2: qmv_pd<K, 2>(pd, grid, st, tr, tiles_n, in, out, xhat, xs, rows, pass_rows, part, suh); break;
-    case 3: qmv_pd<K, 3>(pd, grid, st, tr, tiles_n, in, out, xhat, xs, rows, pass_rows, part, suh); break;
-    default: qmv_pd<K, 4>(pd, grid, st, tr, tiles_n, in, out, xhat, xs, rows, pass_rows, part, suh); break;
+    case 0: qmv_pd<K, 0>(pd, grid, st, tr, tiles_n, in, out, xhat, xs, rows, pass_rows, group, part, suh); break;
+    case 1: qmv_pd<K, 1>(pd, grid, st, tr, tiles_n, in, out, xhat, xs, rows, pass_rows, group, part, suh); break;
+    case 2: qmv_pd<K, 2>(pd, grid, st, tr, tiles_n, in, out, xhat, xs, rows, pass_rows, group, part, suh); break;
+    case 3: qmv_pd<K, 3>(pd, grid, st, tr, tiles_n, in, out, xhat, xs, rows, pass_rows, group, part, suh); break;
+    default: qmv_pd<K, 4>(pd, grid, st, tr, tiles_n, in, out, xhat, xs, rows, pass_rows, group, part, suh); break;
   }
 }
 
@@ -558,7 +575,14 @@ exl3_status launch_qmv(const exl3_trellis_desc &shape, const PtrTable &trellis, 
   const int pr = qmv_pass_rows(rows);
   const int64_t gy = (int64_t)n_slices(k_tiles) * ((rows + pr - 1) / pr);
   if (gy > 65535 || n > 65535) return fail(EXL3_ERR_UNSUPPORTED, "linear launch too large");
-  dim3 grid((unsigned)(out / 128), (unsigned)gy, (unsigned)n);
+  // column blocks per workgroup: 2 or 4 while that leaves 768 workgroups (3 per CU). us per
+  // call with 1, 2, 4 blocks (K6 mul1 4096 x 154880, 9680 workgroups): 133, 122, 119 at 8
+  // rows, 101, 98, 100 at 1; 4096 x 24576 (K4, 1536): 33.5, 30.7, 30.5 at 16 rows, 19.7, 19.0,
+  // 22.6 at 1; 8192 x 4096 at 8 rows (512 workgroups): 15.7, 16.0, 18.2.
+  const int64_t blocks = (int64_t)(out / 128) * gy * n;
+  int group = 1;
+  while (group < 4 && blocks / (2 * group) >= 768) group *= 2;
+  dim3 grid((unsigned)((out / 128 + group - 1) / group), (unsigned)gy, (unsigned)n);
   const int tiles_n = out / 16, pd = prefetch_steps(k_tiles, shape.K);
   // the weight form of the process-wide tuning (the reference's f16 weights by default)
   const int kcb = kernel_cb(shape.codebook, tuning().weight_form);
@@ -566,7 +590,7 @@ exl3_status launch_qmv(const exl3_trellis_desc &shape, const PtrTable &trellis, 
 #define EXL3_K(KK)                                                                        \
   case KK:                                                                                \
     qmv_cb<KK>(kcb, pd, grid, st, trellis, tiles_n, in, out, xhat, x_member_stride, rows, \
-               pr, part, suh);                                                            \
+               pr, group, part, suh);                                                     \
     break;
     EXL3_K(1) EXL3_K(2) EXL3_K(3) EXL3_K(4) EXL3_K(5) EXL3_K(6) EXL3_K(7) EXL3_K(8)
 #undef EXL3_K
