@@ -937,7 +937,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kFold ? 7 :
     r1 += y1;
   } else if (a.shared_kind == exl3m::kSharedDense) {
     if constexpr (kFold) {  // k_shared_gemm's output, summed and rounded
-      const uint32_t v = *reinterpret_cast<const uint32_t *>(a.dsh_dn16 + (int64_t)row * a.H + c);
+      const uint16_t *y = reinterpret_cast<const uint16_t *>(a.dsh_dn) + (int64_t)row * a.H + c;
+      const uint32_t v = *reinterpret_cast<const uint32_t *>(y);
       r0 += lo16(v);
       r1 += hi16(v);
     } else {
@@ -1219,7 +1220,6 @@ MoeArgs make_args(const exl3_moe_layer_s *L, const MoeLayout &m, int64_t N, cons
   a.dsh_gu = (float *)(ws + m.dsh_gu);
   a.dsh_act = (uint16_t *)(ws + m.dsh_act);
   a.dsh_dn = (float *)(ws + m.dsh_dn);
-  a.dsh_dn16 = (uint16_t *)(ws + m.dsh_dn);
   a.xrot = (uint16_t *)(ws + m.xrot);
   a.out = out;
   return a;

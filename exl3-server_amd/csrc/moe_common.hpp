@@ -113,8 +113,7 @@ struct MoeArgs {
                        // output Hadamard (slots P.. = a trellis shared expert)
   float *dsh_gu;       // (2, N, SI, 8): f16 shared gate/up k-split partials
   uint16_t *dsh_act;   // (N, SI): f16 shared expert SwiGLU output
-  float *dsh_dn;       // (N, H, 8): f16 shared down k-split partials
-  uint16_t *dsh_dn16;  // long-run mode: (N, H) f16 output of the f16 shared expert (dsh_dn's memory)
+  float *dsh_dn;       // (N, H, 8): f16 shared down k-split partials (long-run mode: (N, H) f16 outputs)
   uint16_t *out;       // (N, H)
   // Optional hyper-connection mix behind the combine (g5_hc_mix): with hc_out set, the
   // combine also writes hc_out[row][n] = post[n] * out[row] + (comb^T @ residual)[n]

@@ -3,7 +3,7 @@
 //
 //  k_shared_gemm<true>   gate and up of the same columns in one workgroup, SwiGLU at the end
 //                        -> dsh_act (N, SI) f16
-//  k_shared_gemm<false>  down -> dsh_dn16 (N, H) f16, the linear's output, added by the combine
+//  k_shared_gemm<false>  down -> dsh_dn as (N, H) f16, the linear's output, added by the combine
 //
 // Per output the arithmetic is dense_mfma's and its consumers': every k split accumulated
 // from zero by 16x16x32 MFMAs in step order, the splits added in order.
@@ -183,7 +183,8 @@ __global__ __launch_bounds__(64 * WR *WC) __attribute__((amdgpu_waves_per_eu(2, 
       } else {
 #pragma unroll
         for (int n = 0; n < TN; ++n)
-          a.dsh_dn16[(row0 + r) * a.H + cb * kCols + 16 * (wc * TN + n) + l15] = f32_to_f16(Y[m][n][i]);
+          reinterpret_cast<uint16_t *>(a.dsh_dn)[(row0 + r) * a.H + cb * kCols + 16 * (wc * TN + n) + l15] =
+              f32_to_f16(Y[m][n][i]);
       }
     }
 }
