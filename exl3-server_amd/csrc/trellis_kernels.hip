@@ -567,6 +567,29 @@ exl3_status launch_qmv_rows(const exl3_trellis_desc &shape, const RowsPlan &p, c
   return EXL3_OK;
 }
 
+// Column blocks per workgroup of k_qmv (1, 2 or 4) from the call's one-block workgroups and rows
+// a pass: the fewest rounds of 256 CUs times a workgroup's work, g blocks' decode and one
+// rotation (rows / 32 of a block's decode). The rounds weigh most: 4096 x 50176 (K4, 3136
+// workgroups) at 1 row takes 32.4, 34.0, 38.3 us with 1, 2, 4 blocks (13, 7, 4 rounds). At least
+// 768 workgroups stay (3 per CU), and below 8 rows, whose rotation is cheap, 2048 (more than are
+// resident at once): 4096 x 32768 (K4, 2048) 22.5, 23.4, 24.9 at 1 row, 30.7, 30.2, 28.3 at 8;
+// 4096 x 24576 (K4, 1536) 33.3, 30.3, 29.6 at 16; 8192 x 24576 (K3, 3072) 41.5, 39.8, 35.1 at 8;
+// the 4096 x 154880 head (K6, 9680) 96, 94, 94 at 1 row, 110, 104, 104 at 4, 133, 122, 119 at 8.
+static int qmv_group(int64_t blocks, int rows) {
+  int best = 1;
+  double t_best = 0;
+  for (int g = 1; g <= 4; g *= 2) {
+    const int64_t wgs = (blocks + g - 1) / g;
+    if (g > 1 && wgs < (rows < 8 ? 2048 : 768)) break;
+    const double t = (double)((wgs + 255) / 256) * (g + rows / 32.0);
+    if (g == 1 || t < t_best) {
+      t_best = t;
+      best = g;
+    }
+  }
+  return best;
+}
+
 exl3_status launch_qmv(const exl3_trellis_desc &shape, const PtrTable &trellis, int n,
                        const uint16_t *xhat, int64_t x_member_stride, int64_t rows, float *part,
                        hipStream_t st, const PtrTable *suh) {
@@ -575,13 +598,7 @@ exl3_status launch_qmv(const exl3_trellis_desc &shape, const PtrTable &trellis, 
   const int pr = qmv_pass_rows(rows);
   const int64_t gy = (int64_t)n_slices(k_tiles) * ((rows + pr - 1) / pr);
   if (gy > 65535 || n > 65535) return fail(EXL3_ERR_UNSUPPORTED, "linear launch too large");
-  // column blocks per workgroup: 2 or 4 while that leaves 768 workgroups (3 per CU). us per
-  // call with 1, 2, 4 blocks (K6 mul1 4096 x 154880, 9680 workgroups): 133, 122, 119 at 8
-  // rows, 101, 98, 100 at 1; 4096 x 24576 (K4, 1536): 33.5, 30.7, 30.5 at 16 rows, 19.7, 19.0,
-  // 22.6 at 1; 8192 x 4096 at 8 rows (512 workgroups): 15.7, 16.0, 18.2.
-  const int64_t blocks = (int64_t)(out / 128) * gy * n;
-  int group = 1;
-  while (group < 4 && blocks / (2 * group) >= 768) group *= 2;
+  const int group = qmv_group((int64_t)(out / 128) * gy * n, pr);
   dim3 grid((unsigned)((out / 128 + group - 1) / group), (unsigned)gy, (unsigned)n);
   const int tiles_n = out / 16, pd = prefetch_steps(k_tiles, shape.K);
   // the weight form of the process-wide tuning (the reference's f16 weights by default)

@@ -25,12 +25,12 @@ def tensors(in_f, out_f, K, seed=0):
     return words, su, sv
 
 
-# (rows, in, out, K, codebook): k slices x column blocks of 1536 and up take 2 blocks a
-# workgroup, of 3072 and up 4
+# (rows, in, out, K, codebook)
 SHAPES = [
-    (1, 4096, 193 * 128, 4, 2), (16, 896, 221 * 128, 3, 0), (7, 1280, 309 * 128, 6, 1),   # 2, the last alone
-    (8, 1152, 345 * 128, 5, 2), (2, 1152, 342 * 128, 1, 1), (5, 2560, 615 * 128, 8, 0),   # 4, the last 1, 2, 3
-    (3, 1280, 616 * 128, 2, 0), (15, 2048, 768 * 128, 7, 2), (16, 128, 3073 * 128, 4, 1), # 4, the last 4, 4, 1
+    (9, 4096, 192 * 128, 4, 2), (16, 896, 221 * 128, 3, 0), (16, 1280, 309 * 128, 6, 1),   # 2 blocks, the last 2, 1, 1
+    (8, 1152, 345 * 128, 5, 2), (16, 128, 3073 * 128, 4, 1),                               # 2, the last alone
+    (15, 2048, 768 * 128, 7, 2), (2, 1024, 5001 * 128, 1, 1),                              # 4, the last 4, 1
+    (4, 1152, 970 * 128, 8, 0), (3, 256, 8191 * 128, 2, 0),                                # 4, the last 2, 3
 ]
 
 
@@ -54,7 +54,7 @@ def test_groups_of_members():
     # three members of 9 x 59 workgroups each: groups of 2 in the joint launch, none alone
     in_f, out_f, K, cb = 1152, 59 * 128, 4, 1
     ws = [TrellisWeight(*tensors(in_f, out_f, K, s), in_f, out_f, K, cb) for s in (1, 2, 3)]
-    x = torch.randn((6, in_f), device="cuda:0").half()
+    x = torch.randn((16, in_f), device="cuda:0").half()
     y = trellis_linear_group(ws, x)
     for m in range(3):
         assert torch.equal(y[m], trellis_linear(ws[m], x))
