@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstdint>
 #include <utility>
 
 #include "exl3_device.hpp"
@@ -503,6 +504,11 @@ int qmv_pass_rows(int64_t rows) {
 
 int qmv_slices(int in) { return n_slices(in / 16); }
 
+// Waves of k_stage_rows.
+static int64_t stage_waves(int64_t rows, int in, int n) {
+  return (int64_t)n * rows * ((in / 128 + kStageBatch - 1) / kStageBatch);
+}
+
 // The linear's path: the slice-parallel k_qmv (16 rows per decode, f32 slice partials through
 // memory, the rotation repeated by every column block) or k_qmv_rows (64 or 128 rows per
 // decode, the whole k range in one workgroup) in one of its three shapes, whichever is
@@ -518,6 +524,9 @@ RowsPlan rows_plan(int in, int out, int64_t rows, int n) {
   RowsPlan best{};
   // (calls past the slice path's grid limit are refused there)
   if (rows <= 16 || (int64_t)n_slices(in / 16) * ((rows + 15) / 16) > 65535) return best;
+  // k_stage_rows' grid: a launch has at most 2^32 - 1 threads in a dimension (128 members of
+  // 1536 x 128 pass it from 262,144 rows, where the slice path's launches still fit)
+  if (stage_waves(rows, in, n) * 64 > (int64_t)UINT32_MAX - 256) return best;
   const double k = in / 4096.0;
   double t_best = 4.0 + 4.0 * (double)((rows + 15) / 16) * ((double)in * out * n / (1 << 24));
   const struct {
@@ -527,7 +536,7 @@ RowsPlan rows_plan(int in, int out, int64_t rows, int n) {
   for (const auto &s : shapes) {
     const int64_t tiles = (rows + 16 * s.rb - 1) / (16 * s.rb);
     const int64_t wgs = tiles * ((out / 32 + s.waves - 1) / s.waves) * n;
-    if (wgs > 0x7fffffff) continue;
+    if (wgs * s.waves * 64 > (int64_t)UINT32_MAX) continue;
     const double t = 8.0 + k * std::max(s.alone, s.full * (double)((wgs + 255) / 256));
     if (t < t_best) {
       t_best = t;
@@ -539,7 +548,7 @@ RowsPlan rows_plan(int in, int out, int64_t rows, int n) {
 
 exl3_status launch_stage_rows(const uint16_t *x, int64_t x_member_stride, int64_t rows, int in, int n,
                               const PtrTable *suh, uint16_t *xrot, hipStream_t st) {
-  const int64_t waves = (int64_t)n * rows * ((in / 128 + kStageBatch - 1) / kStageBatch);
+  const int64_t waves = stage_waves(rows, in, n);
   k_stage_rows<<<(unsigned)((waves + 3) / 4), 256, 0, st>>>(x, x_member_stride, rows, in, n, suh ? *suh : PtrTable{},
                                                             suh ? 1 : 0, xrot);
   EXL3_LAUNCHED("k_stage_rows");

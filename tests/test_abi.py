@@ -84,6 +84,16 @@ def test_workspace_too_small_is_reported_before_launch():
     assert st == _lib.EXL3_ERR_WORKSPACE
 
 
+def test_workspace_query_of_calls_past_the_row_stagings_grid():
+    # 128 members of 1536 x 128: rotating 262,144 rows beforehand would take 2^32 threads in
+    # one launch, so the call stays on the slice path and asks for its partials (3 k slices);
+    # a row block less, the rotated rows are the larger
+    L = _lib.lib()
+    d = fake_desc(in_f=1536, out_f=128)
+    for rows, per_row in ((262144, 3 * 128 * 4), (262144 - 16, 1536 * 2)):
+        assert L.exl3_trellis_workspace_size(C.byref(d), rows, 128) == 128 * rows * per_row
+
+
 def test_topk_route_rejects_bad_config():
     L = _lib.lib()
     cfg = _lib.MoeConfig(0, 0, 5, 6, 1, 1, 1, 1.0, 0.0)  # top_k > E
