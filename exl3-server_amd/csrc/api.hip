@@ -82,6 +82,15 @@ LinearWs linear_ws(int in, int out, int64_t rows, int n) {
 // Calls of many rows (RowsPlan): the rotated rows (n, rows, in) f16 instead.
 size_t rows_ws(int in, int64_t rows, int n) { return align_up((size_t)n * rows * in * 2, 256); }
 
+// The plan of a call of n members: many rows take k_qmv_rows with reference-form weights and
+// no explicit rows_per_pass.
+RowsPlan call_plan(const exl3_trellis_desc &w, int64_t rows, int n) {
+  const exl3_tuning tn = tuning();
+  const bool reference = tn.weight_form == EXL3_FORM_REFERENCE || w.codebook == EXL3_CB_MUL1;
+  if (!reference || tn.rows_per_pass > 0) return RowsPlan{};
+  return rows_plan(w.in_features, w.out_features, rows, n);
+}
+
 exl3_status check_ws(void *ws, size_t bytes, size_t need) {
   if (need && (!ws || bytes < need))
     return fail(EXL3_ERR_WORKSPACE, "workspace too small: need " + std::to_string(need) +
@@ -105,13 +114,9 @@ exl3_status linear_core(const exl3_trellis_desc *members, int n, const uint16_t 
   float *part = reinterpret_cast<float *>((char *)ws + lw.part_off);
   const int n_sl = qmv_slices(in);
   // many rows: every weight decoded once per rb * 16 rows, over rows rotated beforehand into
-  // the workspace (reference-form weights, no explicit rows_per_pass, outputs and svh aligned
-  // for its paired loads and stores; a workspace that only holds the slice partials keeps
-  // the slice path: the bits are the same)
-  const exl3_tuning tn = tuning();
-  const bool reference = tn.weight_form == EXL3_FORM_REFERENCE || w0.codebook == EXL3_CB_MUL1;
-  RowsPlan plan{};
-  if (reference && tn.rows_per_pass <= 0) plan = rows_plan(in, out, rows, n < PtrTable::kMax ? n : PtrTable::kMax);
+  // the workspace (outputs and svh aligned for its paired loads and stores; a workspace that
+  // only holds the slice partials keeps the slice path: the bits are the same)
+  RowsPlan plan = call_plan(w0, rows, n < PtrTable::kMax ? n : PtrTable::kMax);
   uintptr_t align = reinterpret_cast<uintptr_t>(y16) | reinterpret_cast<uintptr_t>(svh_stack) |
                     (reinterpret_cast<uintptr_t>(y32) & 7 ? 1 : 0);
   if (!svh_stack)
@@ -178,7 +183,9 @@ exl3_status exl3_trellis_path_info(const exl3_trellis_desc *w, int64_t rows,
   if (rc) return rc;
   if (!info || rows < 0) return fail(EXL3_ERR_INVALID, "bad path_info arguments");
   const exl3_tuning tn = tuning();
-  const int mb = qmv_pass_rows(rows);
+  // calls of many rows: 16 * rb rows per decode, the whole k range in one workgroup
+  const RowsPlan plan = call_plan(*w, rows, 1);
+  const int mb = plan.rb ? 16 * plan.rb : qmv_pass_rows(rows);
   // Every pass runs on the matrix cores; "staged" reports the reference's criterion
   // (a pass shared by at least mat_min_rows rows, trellis_gemm.cpp:800-812).
   info->staged = (tn.mat_min_rows > 0 && rows >= tn.mat_min_rows &&
@@ -188,8 +195,8 @@ exl3_status exl3_trellis_path_info(const exl3_trellis_desc *w, int64_t rows,
   info->rows_per_block = mb;
   info->pad_rows = (int32_t)((rows + mb - 1) / mb * mb);
   info->passes = (int32_t)((rows + mb - 1) / mb);
-  info->splits = qmv_slices(w->in_features);
-  info->tiles_per_workgroup = 32;
+  info->splits = plan.rb ? 1 : qmv_slices(w->in_features);
+  info->tiles_per_workgroup = plan.rb ? 8 * plan.waves : 32;
   return EXL3_OK;
 }
 

@@ -113,15 +113,18 @@ typedef enum {
  * the reference, whose Metal QMV has the reference form only) selects the mcg/3inst
  * weights: EXL3_FORM_REFERENCE (0, the default) or EXL3_FORM_HALVES. */
 typedef struct {
-  int32_t rows_per_pass;  /* 0 = auto: min(rows, 16), one MFMA pass */
+  int32_t rows_per_pass;  /* 0 = auto: min(rows, 16), or 64 or 128 in calls of many rows */
   int32_t mat_min_rows;   /* calls of >= this many rows count as staged (default 16) */
   int32_t mat_max_rows;   /* 0 = no cap */
   int32_t weight_form;    /* exl3_weight_form */
 } exl3_tuning;
 
 /* What a trellis linear at `rows` rows will do. Mirrors TrellisPathInfo
- * (trellis_gemm.h:154-162). passes = weight streams per call, counted in MFMA passes of
- * rows_per_block rows (calls of many rows decode a weight once for several of them). */
+ * (trellis_gemm.h:154-162) for a call of one member with the queried workspace and 8-byte
+ * aligned outputs. passes = weight streams per call, of rows_per_block rows each: up to 16
+ * (with the k range in `splits` slices, whose partials go through the workspace), or in
+ * calls of many rows 64 or 128 (splits = 1: the whole k range in one workgroup, added up in
+ * the same slices). tiles_per_workgroup = 16x16 weight tiles of a workgroup's step. */
 typedef struct {
   int32_t staged;
   int32_t rows_per_block;

@@ -84,6 +84,34 @@ def test_workspace_too_small_is_reported_before_launch():
     assert st == _lib.EXL3_ERR_WORKSPACE
 
 
+def test_path_info_of_calls_of_many_rows():
+    def ask(d, rows):
+        info = _lib.PathInfo()
+        _lib.call("exl3_trellis_path_info", C.byref(d), rows, C.byref(info))
+        return info
+
+    d, mul1 = fake_desc(out_f=24576), fake_desc(out_f=24576, cb=2)
+    info = ask(d, 1000)
+    # weights are decoded once per 64 or 128 rows, over the whole k range
+    assert info.rows_per_block in (64, 128) and info.splits == 1 and info.staged == 1
+    assert info.passes == -(-1000 // info.rows_per_block)
+    assert info.pad_rows == info.passes * info.rows_per_block
+    assert info.tiles_per_workgroup in (32, 64)
+    t0 = _lib.Tuning()
+    _lib.call("exl3_get_tuning", C.byref(t0))
+    try:
+        # explicit passes and the halves form keep the slice path; mul1 has one form only
+        _lib.call("exl3_set_tuning", C.byref(_lib.Tuning(8, 16, 0, _lib.FORM_REFERENCE)))
+        info = ask(d, 1000)
+        assert (info.rows_per_block, info.passes, info.splits) == (8, 125, 8)
+        _lib.call("exl3_set_tuning", C.byref(_lib.Tuning(0, 16, 0, _lib.FORM_HALVES)))
+        info = ask(d, 1000)
+        assert (info.rows_per_block, info.passes, info.splits) == (16, 63, 8)
+        assert ask(mul1, 1000).splits == 1
+    finally:
+        _lib.call("exl3_set_tuning", C.byref(t0))
+
+
 def test_workspace_query_of_calls_past_the_row_stagings_grid():
     # 128 members of 1536 x 128: rotating 262,144 rows beforehand would take 2^32 threads in
     # one launch, so the call stays on the slice path and asks for its partials (3 k slices);
