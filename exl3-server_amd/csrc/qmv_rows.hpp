@@ -47,8 +47,11 @@ __device__ __forceinline__ void rows_each(std::integer_sequence<int, I...>, F &&
 // accumulator land on different banks.
 __device__ __forceinline__ int rows_col(int r, int c) { return c ^ (((r >> 2) & 1) << 5) ^ (((r >> 3) & 1) << 3); }
 
+// (Waves per SIMD: the 64-row tile of K <= 4 fits 168 registers. At K = 5 it spilled 16 to 41
+// of them under that bound: 4096 x 24576 at 17 rows took 48.7, 45.2 and 40.6 us by codebook,
+// without spills 42.8, 42.1 and 38.5; the slice path 46.5, 45.8 and 45.9.)
 template <int K, int CB, int RB, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(RB > 4 || K > 5 ? 2 : 3))) void k_qmv_rows(RowsArgs a) {
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(RB > 4 || K > 4 ? 2 : 3))) void k_qmv_rows(RowsArgs a) {
   static_assert(!dup_cb(CB), "reference-form weights");
   constexpr int PD = 2;
   __shared__ __align__(16) uint32_t buf_a[kRowsBufWords<RB>], buf_b[kRowsBufWords<RB>];
