@@ -215,12 +215,24 @@ __global__ __launch_bounds__(256) void k_hadamard(const uint16_t *__restrict__ x
 // Bound by decode VALU, the rotation of the rows beside it: a workgroup rotates its slice of
 // every row whatever its columns, so a group of blocks (kGroup) rotates once for all of them
 // and keeps one ring-word stream over them (waves per SIMD as in the expert kernels).
+// The slice partials of an n-pair's rows below nr, from p (its first row and column).
+__device__ __forceinline__ void qmv_store(float *p, int out, int nr, const f32x4 &D0, const f32x4 &D1) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = d_row(i);
+    if (r < nr) {
+      p[(int64_t)r * out + d_col(0)] = D0[i];
+      p[(int64_t)r * out + d_col(1)] = D1[i];
+    }
+  }
+}
+
 template <int K, int CB, int PD, bool kGroup>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kGroup ? (K <= 4 ? 7 : 6) : 1))) void k_qmv(exl3h::PtrTable trellis, int tiles_n, int in,
                                              int out, const uint16_t *__restrict__ xhat,
                                              int64_t x_member_stride, int64_t rows,
-                                             int pass_rows, int group, float *__restrict__ part,
-                                             exl3h::PtrTable suh, int rotate) {
+                                             int pass_rows, float *__restrict__ part,
+                                             exl3h::PtrTable suh, int rotate, int group) {
   constexpr bool kDup = dup_cb(CB);
   // one ring-word slot per wave, then the slice's staged rows (pass_rows of them: the
   // launch sizes the LDS to the pass, so a one-row call is not held to the occupancy of
@@ -287,27 +299,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kGroup ? (K
     }
   }
   __syncthreads();
-  float *p = part + (((int64_t)member * n_sl + sl) * rows + r0) * out + cb * 128 + wave * 32;
-  const uint32_t *xrow = xs + min(lane & 15, nr - 1) * xs_stride;
-  u32x4 *slot = slots + wave * slot_chunks(K);
-  auto store = [=](int it, const f32x4 &D0, const f32x4 &D1) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = d_row(i);
-      if (r < nr) {
-        float *o = p + (int64_t)r * out + it * 128;
-        o[d_col(0)] = D0[i];
-        o[d_col(1)] = D1[i];
-      }
-    }
-  };
+  // (one block: the output pointer is formed after the decode loop; formed before it, it changed
+  // the loop's schedule, 2048 x 12288 K3 at 17 rows 16.2 to 16.6 us)
   if constexpr (kGroup) {
-    qmv_slice_items<K, CB, PD>(S, ss, min(group, out / 128 - cb), xrow, slot, store);
+    float *p = part + (((int64_t)member * n_sl + sl) * rows + r0) * out + cb * 128 + wave * 32;
+    qmv_slice_items<K, CB, PD>(S, ss, min(group, out / 128 - cb), xs + min(lane & 15, nr - 1) * xs_stride,
+                               slots + wave * slot_chunks(K), [=](int it, const f32x4 &D0, const f32x4 &D1) {
+                                 qmv_store(p + it * 128, out, nr, D0, D1);
+                               });
   } else {
     f32x4 D0, D1;
     qmv_slice<K, CB, PD>((const uint32_t *)trellis.p[member], k_tiles, tiles_n, sl * kStepTiles * ss, cb * 4 + wave,
-                         ss, xrow, slot, D0, D1);
-    store(0, D0, D1);
+                         ss, xs + min(lane & 15, nr - 1) * xs_stride, slots + wave * slot_chunks(K), D0, D1);
+    float *p = part + (((int64_t)member * n_sl + sl) * rows + r0) * out + cb * 128 + wave * 32;
+    qmv_store(p, out, nr, D0, D1);
   }
 }
 
@@ -465,8 +470,8 @@ static void qmv_go(dim3 grid, hipStream_t st, const PtrTable &tr, int tiles_n, i
   const size_t lds = (size_t)4 * slot_chunks(K) * 16 +
                      (size_t)pass_rows * staged_row_words(in / 16, dup_cb(CB)) * 4;
   const auto k = group > 1 ? k_qmv<K, CB, PD, true> : k_qmv<K, CB, PD, false>;
-  k<<<grid, 256, lds, st>>>(tr, tiles_n, in, out, xhat, xs, rows, pass_rows, group, part, suh ? *suh : PtrTable{},
-                            suh ? 1 : 0);
+  k<<<grid, 256, lds, st>>>(tr, tiles_n, in, out, xhat, xs, rows, pass_rows, part, suh ? *suh : PtrTable{},
+                            suh ? 1 : 0, group);
 }
 
 template <int K, int CB>
