@@ -50,6 +50,13 @@ constexpr int kHcRows = 16;       // positions per row tile (the MFMA's rows)
 // group at 256 positions, 17.9 against 17.7 at 384, 68 against 47 at 2048; at 64, 10.6 against
 // 15.1. (256 positions of one 512-wide stream: 9.0 against 10.9.)
 constexpr int kHcManyRows = 384;
+// Calls of few positions and more than 4 streams: a wave's chunk is 48 to 80 dependent-issue
+// MFMAs (3 to 5 tiles of projections). While the call has at most this many workgroups of all
+// tiles, one per CU, each tile gets a workgroup of its own. Both kernels, 8 streams: 11.5 us
+// against 9.5 at one position of 1024 (32 workgroups), 22.6 against 21.6 at 16 of 8192 (256),
+// but 19.8 against 20.7 at 64 of 4096 (512); 5 streams of 512 at 383 positions (240) 11.1 either
+// way. (A thread per projection, before: 10.4 at one position of 8 x 1024.)
+constexpr int kHcSplitGroups = 256;
 
 // Values per (position, partial): the W = (2+N)*N projections' bound (kN = 4: 1..4
 // streams; kN = 8: 5..8), then the sum of squares at index kMaxW.
@@ -137,7 +144,7 @@ __device__ __forceinline__ void hc_chunk(const HcChunkRegs<NT, RT> &c, f32x4 (&E
 // own row of the streams, took 474; two row tiles per wave, so that a loaded fn value serves 32
 // positions: 30.8 against 36 for one, and 33 for four (one wave per SIMD). At 4 positions both
 // forms are a round of loads: 4.6 us.
-// Workgroup (slice, RT row tiles): 4 waves of kC consecutive chunks each (kC = 1: the slice
+// Workgroup (slice, RT row tiles, tiles of projections from NT * blockIdx.z): 4 waves of kC consecutive chunks each (kC = 1: the slice
 // is a group; kC = 4: a super-group), every chunk's loads issued one chunk ahead, then the
 // waves' sums added in order through LDS.
 template <int kN, int NT, int RT, int kC>
@@ -151,6 +158,7 @@ __global__ __launch_bounds__(64 * kHcWaves) void k_hc_proj(const uint16_t *__res
   const int slice = blockIdx.x, lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t p0 = (int64_t)blockIdx.y * (kHcRows * RT);
+  const int j0 = 16 * NT * (int)blockIdx.z;  // this workgroup's first projection
   const int chunks = ND / kHcChunk;
   const int c0 = (slice * kHcWaves + wave) * kC;
   const int n = min(kC, chunks - c0);                                          // this wave's chunks
@@ -162,7 +170,7 @@ __global__ __launch_bounds__(64 * kHcWaves) void k_hc_proj(const uint16_t *__res
 #pragma unroll
   for (int r = 0; r < RT; ++r) srow[r] = streams + min<int64_t>(p0 + 16 * r + c, P - 1) * ND + 8 * g;
 #pragma unroll
-  for (int t = 0; t < NT; ++t) frow[t] = fn + (int64_t)min(16 * t + c, W - 1) * ND + 8 * g;
+  for (int t = 0; t < NT; ++t) frow[t] = fn + (int64_t)min(j0 + 16 * t + c, W - 1) * ND + 8 * g;
   f32x4 D[RT][NT];
   float sq[RT];
   if (n > 0) {
@@ -216,10 +224,10 @@ __global__ __launch_bounds__(64 * kHcWaves) void k_hc_proj(const uint16_t *__res
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const int64_t p = p0 + 16 * rr + 4 * g + k;
-      if (p < P && 16 * t + c < W) part[(p * gridDim.x + slice) * kVals + 16 * t + c] = v[k];
+      if (p < P && j0 + 16 * t + c < W) part[(p * gridDim.x + slice) * kVals + j0 + 16 * t + c] = v[k];
     }
   }
-  if (wave < RT) {
+  if (wave < RT && j0 == 0) {
     float v = s_q[0][wave][lane];
     for (int w = 1; w < n_waves; ++w) v = v + s_q[w][wave][lane];
     if constexpr (kC == 1) {
@@ -620,12 +628,15 @@ static void hc_proj_go(bool many, const uint16_t *streams, int64_t P, int ND, in
                        int n_slices, hipStream_t st) {
   // (5 tiles of projections: one row tile per wave, within the registers of two waves a SIMD)
   constexpr int RT = NT <= 3 ? 2 : 1;
+  const unsigned tiles = (unsigned)((P + kHcRows - 1) / kHcRows);
   if (many)
     k_hc_proj<kN, NT, RT, kHcFan><<<dim3((unsigned)n_slices, (unsigned)((P + kHcRows * RT - 1) / (kHcRows * RT))),
                                     64 * kHcWaves, 0, st>>>(streams, P, ND, W, fn, part);
+  else if (NT > 2 && (int64_t)n_slices * tiles <= kHcSplitGroups)
+    k_hc_proj<kN, 1, 1, 1><<<dim3((unsigned)n_slices, tiles, (unsigned)NT), 64 * kHcWaves, 0, st>>>(streams, P, ND, W,
+                                                                                                fn, part);
   else
-    k_hc_proj<kN, NT, 1, 1><<<dim3((unsigned)n_slices, (unsigned)((P + kHcRows - 1) / kHcRows)), 64 * kHcWaves, 0,
-                              st>>>(streams, P, ND, W, fn, part);
+    k_hc_proj<kN, NT, 1, 1><<<dim3((unsigned)n_slices, tiles), 64 * kHcWaves, 0, st>>>(streams, P, ND, W, fn, part);
 }
 
 template <int kN>

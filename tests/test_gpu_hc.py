@@ -335,6 +335,31 @@ def test_hc_prepare_many_positions(oracle, dev, P, N, D):
     assert torch.equal(hc_prepare(d, site, nw, NORM_EPS)[0], rms_norm(out, nw, NORM_EPS))
 
 
+# More than 4 streams, few positions: a workgroup per tile of projections up to 256 workgroups
+# of all tiles, all tiles in one above. Either side of that (16 and 17 positions of 8 x 8192,
+# 240 and 256 of 5 x 1024 against 272), every count of tiles, a last tile of 3 to 16.
+@pytest.mark.parametrize("P,N,D", [(16, 8, 8192), (17, 8, 8192), (5, 5, 64), (200, 5, 1024), (272, 5, 1024),
+                                   (31, 6, 704), (40, 7, 576), (33, 8, 1024)])
+def test_hc_prepare_tiles_of_projections(oracle, dev, P, N, D):
+    fn, base, scale = make_site(7 * P + N, N, D)
+    st = streams_of(P + D + 1, P, N, D)
+    site = DeviceHcSite.from_numpy(fn, base, scale, N, 20, EPS, dev)
+    d = dev_f16(st, dev)
+    out, post, comb = hc_prepare(d, site, None)
+    rows = [0, P // 2, P - 1]
+    _, opost, ocomb = oracle.hc_prepare(np.ascontiguousarray(st[rows]), N, D, fn, base, scale, 20, EPS)
+    # the bounds of test_hc_prepare_vs_oracle
+    assert np.max(np.abs(post.cpu().numpy()[rows] - opost)) <= 2e-5
+    assert np.max(np.abs(comb.cpu().numpy()[rows] - ocomb)) <= 2e-5
+    for r in rows:
+        one = hc_prepare(d[r:r + 1].contiguous(), site, None)
+        assert all(torch.equal(a[0], b[r]) for a, b in zip(one, (out, post, comb)))
+    # the many-position form on the same rows
+    n = -(-400 // P)
+    many = hc_prepare(d.repeat(n, 1, 1), site, None)
+    assert all(torch.equal(a[:P], b) for a, b in zip(many, (out, post, comb)))
+
+
 @pytest.mark.parametrize("D", [2, 6, 130, 2046, 2050, 4094, 4098, 8190])
 def test_rms_norm_ragged_hidden(oracle, dev, D):
     # rows that are no multiple of the kernel's 8-value vectors, either side of its vector
