@@ -457,8 +457,15 @@ __device__ __forceinline__ int long_item(int b, int per_unit, int shared_mode, c
   return x * q + min(x, r) + (b >> 3);
 }
 
+// Waves per SIMD: 4, that is 128 registers; 3 for the instances that need 130 to 138. 48 experts
+// of 4096 x 1024 at 200 rows: K1 3inst 155 us with 22 registers spilled, 137 without; mcg K2,
+// K3 and K8, 6 to 8 spilled, 136, 139 and 165 against 134, 139 and 163.
+constexpr int gu_long_waves(int K, int CB) {
+  return (K == 1 && CB == 0) || ((K == 2 || K == 3 || K == 8) && CB == 1) ? 3 : 4;
+}
+
 template <int K, int CB, int PD>
-__global__ __launch_bounds__(long_threads(dup_cb(CB))) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_moe_gate_up_long(MoeArgs a, int shared_mode, int) {
+__global__ __launch_bounds__(long_threads(dup_cb(CB))) __attribute__((amdgpu_waves_per_eu(gu_long_waves(K, CB), 8))) void k_moe_gate_up_long(MoeArgs a, int shared_mode, int) {
   extern __shared__ uint32_t smem[];
   constexpr int kWaves = long_threads(dup_cb(CB)) / 64;
   const int out = shared_mode ? a.SI : a.I;
