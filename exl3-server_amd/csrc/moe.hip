@@ -30,6 +30,7 @@ exl3_status launch_moe_expert(int which, int K, int cb, int64_t runs, const MoeA
 int moe_slices(int in);
 exl3_status launch_moe_act(const MoeArgs &a, int shared_mode, int dense_blocks, hipStream_t st);
 exl3_status launch_moe_rotate(const MoeArgs &a, int64_t slot0, int64_t n_slots, hipStream_t st);
+bool shared_products(int64_t N, int H, int SI, int I, int E, int topk);
 exl3_status launch_shared_dense(MoeArgs a, hipStream_t st);
 }
 
@@ -823,8 +824,8 @@ __device__ __forceinline__ void down_out(float2 y, uint32_t sv, float &y0, float
 
 // kFold: a long-run call (one folded down partial per slot, a.fold). Its variant holds
 // few enough VGPRs for 7 waves per SIMD (the general one: 4), so that many more rows'
-// loads are in flight over a long call's many rows; the f16 shared expert's output is then
-// one f16 value, loaded after the ranks.
+// loads are in flight over a long call's many rows; the f16 shared expert's output (one f16
+// value) or its partials are then loaded after the ranks.
 template <bool kFold>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kFold ? 7 : 1))) void k_moe_combine(MoeArgs a) {
   const int lane = threadIdx.x & 63;
@@ -935,27 +936,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kFold ? 7 :
     down_out(ys, *reinterpret_cast<const uint32_t *>(a.svh_s[2] + (int64_t)a.E * a.H + c), y0, y1);
     r0 += y0;
     r1 += y1;
+  } else if (kFold && a.shared_kind == exl3m::kSharedProducts) {  // summed and rounded
+    const uint16_t *y = reinterpret_cast<const uint16_t *>(a.dsh_dn) + (int64_t)row * a.H + c;
+    const uint32_t v = *reinterpret_cast<const uint32_t *>(y);
+    r0 += lo16(v);
+    r1 += hi16(v);
   } else if (a.shared_kind == exl3m::kSharedDense) {
-    if constexpr (kFold) {  // k_shared_gemm's output, summed and rounded
-      const uint16_t *y = reinterpret_cast<const uint16_t *>(a.dsh_dn) + (int64_t)row * a.H + c;
-      const uint32_t v = *reinterpret_cast<const uint32_t *>(y);
-      r0 += lo16(v);
-      r1 += hi16(v);
-    } else {
-      // dense_slots_sum's order over the two outputs' kDenseSlots partials
-      const int S = dense_mfma_splits(a.SI);
-      const float v0[8] = {dsh[0].x, dsh[0].y, dsh[0].z, dsh[0].w, dsh[1].x, dsh[1].y, dsh[1].z, dsh[1].w};
-      const float v1[8] = {dsh[2].x, dsh[2].y, dsh[2].z, dsh[2].w, dsh[3].x, dsh[3].y, dsh[3].z, dsh[3].w};
-      float d0 = v0[0], d1 = v1[0];
+    if (kFold) load_dsh();
+    // dense_slots_sum's order over the two outputs' kDenseSlots partials
+    const int S = dense_mfma_splits(a.SI);
+    const float v0[8] = {dsh[0].x, dsh[0].y, dsh[0].z, dsh[0].w, dsh[1].x, dsh[1].y, dsh[1].z, dsh[1].w};
+    const float v1[8] = {dsh[2].x, dsh[2].y, dsh[2].z, dsh[2].w, dsh[3].x, dsh[3].y, dsh[3].z, dsh[3].w};
+    float d0 = v0[0], d1 = v1[0];
 #pragma unroll
-      for (int q = 1; q < 8; ++q)
-        if (q < S) {
-          d0 += v0[q];
-          d1 += v1[q];
-        }
-      r0 += rf16(d0);
-      r1 += rf16(d1);
-    }
+    for (int q = 1; q < 8; ++q)
+      if (q < S) {
+        d0 += v0[q];
+        d1 += v1[q];
+      }
+    r0 += rf16(d0);
+    r1 += rf16(d1);
   }
   const uint32_t o = pack_f16x2(r0, r1);
   *reinterpret_cast<uint32_t *>(a.out + (int64_t)row * a.H + c) = o;
@@ -1180,6 +1180,9 @@ MoeArgs make_args(const exl3_moe_layer_s *L, const MoeLayout &m, int64_t N, cons
   a.routed_scaling_factor = L->cfg.routed_scaling_factor;
   a.swiglu_limit = L->cfg.swiglu_limit;
   a.shared_kind = L->shared;
+  if (L->shared == exl3m::kSharedDense && N >= long_min_rows() &&
+      shared_products(N, L->H, L->SI, L->I, L->E, L->topk))
+    a.shared_kind = exl3m::kSharedProducts;
   a.logit_splits = dense_mfma_splits(a.H);
   a.n_logit_blocks = (int)dense_mfma_tasks(N, a.H, a.E);  // one task per workgroup
   a.fold = N >= long_min_rows();  // long runs: kLongRows-row passes, slices folded
@@ -1834,10 +1837,8 @@ exl3_status moe_layer_run(exl3_moe_layer_t layer, const uint16_t *h, int64_t N, 
     layer->ev_made = true;
   }
   const int H = layer->H;
-  const bool dense_sh = layer->shared == exl3m::kSharedDense;
-  // the f16 shared expert: as tasks inside the expert launches, or (long-run calls) as two
-  // matrix products
-  const bool dense_tasks = dense_sh && !a.fold;
+  // the f16 shared expert: as tasks inside the expert launches, or as two matrix products
+  const bool dense_tasks = a.shared_kind == exl3m::kSharedDense;
   const bool trellis_sh = layer->shared == exl3m::kSharedTrellis;
   const int64_t units = a.fold ? m.max_passes : m.R;  // work units: runs or long-run passes
   // Long-run calls: a trellis shared expert (under one wave of the machine on its own)
@@ -1886,7 +1887,7 @@ exl3_status moe_layer_run(exl3_moe_layer_t layer, const uint16_t *h, int64_t N, 
     const hipError_t e = hipEventRecord(layer->ev[1], st);
     if (e != hipSuccess) return fail_joined(hip_check(e, "hipEventRecord"));
   }
-  if (dense_sh && a.fold) {
+  if (a.shared_kind == exl3m::kSharedProducts) {
     rc = launch_shared_dense(a, st);
     if (rc) return fail_joined(rc);
   }

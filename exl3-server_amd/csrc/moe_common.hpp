@@ -17,8 +17,8 @@
 // A trellis shared expert runs the gate/up, act and down kernels on one extra "run"
 // that holds every token row (three more launches; in long-run calls on the layer's
 // second stream, forked after the dispatch and joined before L6).
-// In long-run calls the f16 shared expert is two tiled matrix products before L3
-// (moe_shared.hip) instead of workgroups of L3, L4 and L5.
+// In long-run calls whose f16 shared expert is large it is two tiled matrix products before
+// L3 (moe_shared.hip) instead of workgroups of L3, L4 and L5.
 // Calls of 32 rows or more add k_moe_rotate before L3 (each slot's gate/up input
 // rotated once); calls of 65 rows or more take the long-run gate/up and down kernels
 // over the pass table, and calls of 256 rows or more the tiled router logits kernel.
@@ -49,7 +49,9 @@ struct alignas(16) RunRec {
   const void *p[6];
 };
 
-enum SharedKind { kSharedNone = 0, kSharedTrellis = 1, kSharedDense = 2 };
+// kSharedProducts (MoeArgs only): the f16 shared expert of a long-run call as two matrix
+// products (moe_shared.hip) instead of tasks inside the expert launches.
+enum SharedKind { kSharedNone = 0, kSharedTrellis = 1, kSharedDense = 2, kSharedProducts = 3 };
 
 // Everything a kernel of one layer call needs, passed by value.
 // Long-run mode (calls of at least EXL3_MOE_LONG_ROWS token rows, 65 by default): the
@@ -113,7 +115,7 @@ struct MoeArgs {
                        // output Hadamard (slots P.. = a trellis shared expert)
   float *dsh_gu;       // (2, N, SI, 8): f16 shared gate/up k-split partials
   uint16_t *dsh_act;   // (N, SI): f16 shared expert SwiGLU output
-  float *dsh_dn;       // (N, H, 8): f16 shared down k-split partials (long-run mode: (N, H) f16 outputs)
+  float *dsh_dn;       // (N, H, 8): f16 shared down k-split partials (kSharedProducts: (N, H) f16 outputs)
   uint16_t *out;       // (N, H)
   // Optional hyper-connection mix behind the combine (g5_hc_mix): with hc_out set, the
   // combine also writes hc_out[row][n] = post[n] * out[row] + (comb^T @ residual)[n]

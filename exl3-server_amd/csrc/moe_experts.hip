@@ -207,8 +207,8 @@ static int moe_prefetch(int k_tiles, int K) {
 // which: 0 = gate/up, 1 = down, over `runs` runs (routed: the dispatch's run table,
 // bounded by R; shared_mode 1: the one trellis-shared run). cb is the kernel codebook
 // (kernel_cb: the tensor codebook under the handle's weight form). dense: prepend the f16
-// shared expert's workgroups for this projection (short-run kernels only: whole z planes of
-// the 3-D grid, the workgroups past the shared expert's tasks return at once).
+// shared expert's workgroups for this projection (short-run kernels: whole z planes of the
+// 3-D grid, the workgroups past the shared expert's tasks return at once).
 exl3_status launch_moe_expert(int which, int K, int cb, int64_t runs, const MoeArgs &a,
                               int shared_mode, bool dense, hipStream_t st) {
   const int in = which == 0 ? a.H : (shared_mode ? a.SI : a.I);
@@ -232,6 +232,7 @@ exl3_status launch_moe_expert(int which, int K, int cb, int64_t runs, const MoeA
   dim3 ub;
   int dense_arg = dense_blocks;
   if (a.fold) {
+    blocks += dense_blocks;
     if (blocks == 0) return EXL3_OK;
     if (blocks > 0x7fffffff) return fail(EXL3_ERR_UNSUPPORTED, "expert launch too large");
     ub = dim3((unsigned)blocks);

@@ -465,13 +465,17 @@ constexpr int gu_long_waves(int K, int CB) {
 }
 
 template <int K, int CB, int PD>
-__global__ __launch_bounds__(long_threads(dup_cb(CB))) __attribute__((amdgpu_waves_per_eu(gu_long_waves(K, CB), 8))) void k_moe_gate_up_long(MoeArgs a, int shared_mode, int) {
+__global__ __launch_bounds__(long_threads(dup_cb(CB))) __attribute__((amdgpu_waves_per_eu(gu_long_waves(K, CB), 8))) void k_moe_gate_up_long(MoeArgs a, int shared_mode, int dense_blocks) {
   extern __shared__ uint32_t smem[];
   constexpr int kWaves = long_threads(dup_cb(CB)) / 64;
+  if ((int)blockIdx.x < dense_blocks) {
+    shared_gate_up_block(a.h, a.N, a.H, a.SI, a.sh_dense[0], a.sh_dense[1], a.dsh_gu, blockIdx.x, kWaves);
+    return;
+  }
   const int out = shared_mode ? a.SI : a.I;
   const int n_np = out / 32, n_cb = (n_np + kWaves - 1) / kWaves;
   const int k_tiles = a.H / 16, ss = slice_steps(k_tiles), n_sl = n_slices(k_tiles);
-  int b = long_item(blockIdx.x, 2 * n_cb, shared_mode, a);
+  int b = long_item(blockIdx.x - dense_blocks, 2 * n_cb, shared_mode, a);
   if (b < 0) return;
   const int cb = b % n_cb;
   b /= n_cb;
@@ -543,13 +547,17 @@ __global__ __launch_bounds__(long_threads(dup_cb(CB))) __attribute__((amdgpu_wav
 }
 
 template <int K, int CB, int PD>
-__global__ __launch_bounds__(long_threads(dup_cb(CB))) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_moe_down_long(MoeArgs a, int shared_mode, int) {
+__global__ __launch_bounds__(long_threads(dup_cb(CB))) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_moe_down_long(MoeArgs a, int shared_mode, int dense_blocks) {
   extern __shared__ uint32_t smem[];
   constexpr int kWaves = long_threads(dup_cb(CB)) / 64;
+  if ((int)blockIdx.x < dense_blocks) {
+    shared_down_block(a.dsh_act, a.N, a.H, a.SI, a.sh_dense[2], a.dsh_dn, blockIdx.x, kWaves);
+    return;
+  }
   const int in = shared_mode ? a.SI : a.I;
   const int n_np = a.H / 32, n_cb = (n_np + kWaves - 1) / kWaves;
   const int k_tiles = in / 16, ss = slice_steps(k_tiles), n_sl = n_slices(k_tiles);
-  const int b = long_item(blockIdx.x, n_cb, shared_mode, a);
+  const int b = long_item(blockIdx.x - dense_blocks, n_cb, shared_mode, a);
   if (b < 0) return;
   const int cb = b % n_cb, u = b / n_cb;
   RunInfo ri;

@@ -1,4 +1,4 @@
-// The f16 shared expert of long-run calls (g5_linear's mx::matmul branch, glm5_kda.cpp:120;
+// The f16 shared expert of long-run calls with enough of it (g5_linear's mx::matmul branch, glm5_kda.cpp:120;
 // SwiGLU as in glm5_moe.cpp:66-74): two tiled f16 matrix products, gfx950.
 //
 //  k_shared_gemm<true>   gate and up of the same columns in one workgroup, SwiGLU at the end
@@ -16,6 +16,8 @@
 // another card, 483 to 469).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "exl3_device.hpp"
@@ -200,6 +202,28 @@ static void shared_go(const MoeArgs &a, hipStream_t st) {
 }  // namespace exl3d
 
 namespace exl3h {
+
+using exl3m::kLongRows;
+
+// The f16 shared expert as wave tasks (dense_mfma: 16 rows x 16 outputs x one k split) beside
+// the experts' workgroups, or as the two products, each a chain of k parts of its own, as long
+// for a narrow intermediate. Tasks up to one set of resident waves (4 per SIMD), unless they
+// push more than an eighth of a set of the gate/up launch's expert waves (their number at
+// uniform routing) into a second round. What the shared expert adds to a call, us, tasks
+// against products, by hidden, intermediate and rows:
+//   2048, 128, 70 (1280 tasks) 2, 13       512, 128, 200 (1248) 5, 8     4096, 256, 70 (3840) 12, 21
+//   2048, 384, 100 beside 64 experts of 512 (2688 gate/up tasks, 2028 expert waves) 18, 14
+//   3072, 128, 100 beside 160 of 384 (896, 3530) 6, 18
+//   1024, 256, 200 (4992) 14, 11           2048, 256, 130 (4608) 20, 12  (8-wave workgroups)
+constexpr int64_t kResidentWaves = 4096;
+
+bool shared_products(int64_t N, int H, int SI, int I, int E, int topk) {
+  const int64_t gu = 2 * exl3d::dense_mfma_tasks(N, H, SI);
+  if (gu + exl3d::dense_mfma_tasks(N, SI, H) > kResidentWaves) return true;
+  const double distinct = E * (1.0 - std::pow(1.0 - (double)topk / E, (double)N));
+  const double experts = std::max(distinct, (double)N * topk / kLongRows) * 2 * (I / 32);
+  return experts <= kResidentWaves && experts + gu > kResidentWaves + kResidentWaves / 8;
+}
 
 // Rows from which the 128 x 128 tiles (8 waves) take over from the 64 x 64 ones (4): hidden
 // 4096, intermediate 1024, the two products at 500 rows 35 us in small tiles against 54 in
