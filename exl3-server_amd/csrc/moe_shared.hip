@@ -225,11 +225,15 @@ bool shared_products(int64_t N, int H, int SI, int I, int E, int topk) {
   return experts <= kResidentWaves && experts + gu > kResidentWaves + kResidentWaves / 8;
 }
 
-// Rows from which the 128 x 128 tiles (8 waves) take over from the 64 x 64 ones (4): hidden
-// 4096, intermediate 1024, the two products at 500 rows 35 us in small tiles against 54 in
-// big ones, which leave most CUs idle; the call at 1000 rows 867 against 864; at 2048 rows
-// the products 104 against 78.
-constexpr int kSharedBigRows = 1024;
+// 128 x 128 tiles (8 waves, one workgroup per CU) or 64 x 64 ones (4 waves, two per CU), for each
+// product by its rounds of workgroups: a round of big tiles takes about 1.5 of small ones.
+// Both products with the rest of a small layer, us, small against big tiles, by hidden and
+// intermediate: 4096, 128 at 1024 rows 137, 152 and at 2048 180, 191; 512, 1024 at 1024 65, 72;
+// 2048, 1024 at 1100 121, 116; 4096, 1024 at 2048 234, 222; 4096, 2048 at 1000 197, 181.
+static bool big_tiles(int64_t rows, int64_t cols) {
+  const int64_t big = (rows + 127) / 128 * (cols / 128), small = (rows + 63) / 64 * (cols / 64);
+  return 3 * ((big + 255) / 256) < 2 * ((small + 511) / 512);
+}
 
 exl3_status launch_shared_dense(exl3m::MoeArgs a, hipStream_t st) {
   if (reinterpret_cast<uintptr_t>(a.h) % 4) {
@@ -239,13 +243,10 @@ exl3_status launch_shared_dense(exl3m::MoeArgs a, hipStream_t st) {
     EXL3_HIP(hipMemcpyAsync(x, a.h, (size_t)a.N * a.H * 2, hipMemcpyDeviceToDevice, st));
     a.h = x;
   }
-  if (a.N >= kSharedBigRows) {
-    exl3d::shared_go<true, 4, 2, 2, 4>(a, st);
-    exl3d::shared_go<false, 4, 2, 2, 4>(a, st);
-  } else {
-    exl3d::shared_go<true, 2, 2, 2, 2>(a, st);
-    exl3d::shared_go<false, 2, 2, 2, 2>(a, st);
-  }
+  if (big_tiles(a.N, 2 * (int64_t)a.SI)) exl3d::shared_go<true, 4, 2, 2, 4>(a, st);
+  else exl3d::shared_go<true, 2, 2, 2, 2>(a, st);
+  if (big_tiles(a.N, a.H)) exl3d::shared_go<false, 4, 2, 2, 4>(a, st);
+  else exl3d::shared_go<false, 2, 2, 2, 2>(a, st);
   EXL3_LAUNCHED("k_shared_gemm");
   return EXL3_OK;
 }

@@ -5,9 +5,10 @@ the same arithmetic.
 The routed experts' part of an output differs between the two paths in f32 round-off, so the
 shared expert is isolated: every routed svh is zero, which makes each routed term exactly
 zero, and a row's output is the shared expert's alone. It must then have the bits of a
-short-run call on that row. Sizes, in either form: row tiles of 64 and 128 (from 1024 rows),
-hidden and intermediate sizes whose k splits are 1, 2, 4 and 8 and whose 64-wide parts leave
-remainders; 4096 tasks and the next count that can be.
+short-run call on that row. Sizes, in either form: output tiles of 64 and of 128 (a product of
+more than 512 small ones) for both products and for one, hidden and intermediate sizes whose k
+splits are 1, 2, 4 and 8 and whose 64-wide parts leave remainders; 4096 tasks and the next
+count that can be.
 """
 import numpy as np
 import pytest
@@ -30,7 +31,8 @@ TASKS = [(65, 128, 128), (127, 384, 256), (128, 512, 640), (129, 1024, 128), (20
          (1100, 256, 128), (128, 2048, 384)]
 PRODUCTS = [(1023, 256, 512), (1024, 640, 256), (1025, 2048, 1024), (1100, 1280, 128), (1151, 384, 1152),
             (129, 2048, 384), (65, 4096, 512), (127, 3072, 640), (200, 1792, 1152), (600, 1152, 384),
-            (1000, 640, 640), (1024, 1024, 256)]
+            (1000, 640, 640), (1024, 1024, 256), (1151, 1920, 1152), (1500, 1280, 1152), (2000, 1152, 896),
+            (1030, 2048, 256)]
 
 
 @pytest.mark.parametrize("rows,H,SI", TASKS + PRODUCTS)
