@@ -10,8 +10,8 @@ namespace {
 
 // Long-run mode: the input Hadamard of every (slot, projection) once, x_rot[slot][proj]
 // = had_pre(h[row], suh of the slot's expert and projection) in the staged k order, so
-// the gate/up workgroups of a pass (one per 256 output columns) copy it instead of each
-// rotating it again. One wave per (slot, projection), kRotBatch 128-blocks at a time;
+// the gate/up workgroups of a pass (one per 128 output columns, 256 in the halves form) copy
+// it instead of each rotating it again. One wave per (slot, projection), kRotBatch 128-blocks at a time;
 // slots [slot0, slot0 + n_slots): routed slots (below P, from the dispatch) or the N
 // shared slots of a trellis shared expert (slot P + i is token row i, whatever the
 // routing: so they can be rotated before the dispatch has run).

@@ -261,7 +261,7 @@ __global__ __launch_bounds__(kDnThreads) __attribute__((amdgpu_waves_per_eu(kDnW
 
 // Long runs (calls of 65 token rows or more): workgroups of 4 waves (8 in the halves form),
 // wave w owns n-pair 4*cb + w, passes of up to kLongRows rows with up to kLongBlocks 16-row MFMA blocks
-// per decode (qmv_slice_rb over the pass's occupied blocks only), and every k slice of
+// per decode (over the pass's occupied blocks only), and every k slice of
 // the tensor in one workgroup: each block's accumulators run on from the first k step
 // to the last (the reference's staged path likewise sums in its own association, within
 // 1% of max |value| of its QMV by its test, glm5_gemv_nt_test.cpp:221-247). One partial
@@ -272,20 +272,17 @@ using exl3m::kLongRows;
 // staged rows; in the reference form 4 measured as fast as 8, and 2% faster at 100 rows).
 constexpr int long_threads(bool dup) { return dup ? 512 : 256; }
 constexpr int kStageThreads = long_threads(true);  // stage_part's (halves form)
-// Staging loads in flight per lane: a slice of 64 plain rows is 64 x 64 chunks, 8 per
-// thread (two rounds of 4); a 4-step part of duplicated rows (the halves form) 64 x 32,
-// 4 per thread (one round).
-constexpr int kStageBatchGu = 4;
-constexpr int kStageBatchDn = 4;
+// Its staging loads in flight per lane: a 4-step part of duplicated rows is 64 x 32 chunks, 4
+// per thread (one round).
+constexpr int kStageBatch = 4;
 
-// Stages one part of a pass's rows into LDS: rows [0, nr) of the source, row r at byte
+// Halves form: stages one part of a pass's rows into LDS: rows [0, nr) of the source, row r at byte
 // r * row_bytes of `src` (a buffer resource that covers exactly those nr rows), their
 // 16-byte chunks [kbyte0 / 16, kbyte0 / 16 + q_row) into staged rows xs + r * xs_stride.
 // Thread t takes chunk t % q_row of rows t / q_row + j * (kStageThreads / q_row) (q_row a
 // power of two that divides kStageThreads), so that its source offset and LDS row only
-// step by whole rows; kBatch loads are issued before the first LDS store. A load of a row
+// step by whole rows; kStageBatch loads are issued before the first LDS store. A load of a row
 // at or past nr falls outside the resource and reads zero (no address clamps).
-template <bool kDup, int kBatch>
 __device__ __forceinline__ void stage_part(__amdgpu_buffer_rsrc_t src, uint32_t row_bytes, uint32_t kbyte0,
                                            int q_row, int q_lg, int nr, uint32_t *xs, int xs_stride) {
   // the thread's offsets are derived afresh at each call (the empty volatile asm keeps the
@@ -300,16 +297,16 @@ __device__ __forceinline__ void stage_part(__amdgpu_buffer_rsrc_t src, uint32_t 
   uint32_t vo = (uint32_t)r0 * row_bytes + (uint32_t)cq * 16 + kbyte0;
   uint32_t *dst = xs + r0 * xs_stride;
   const int dstep = rstep * xs_stride;
-  for (int r = r0; r < nr; r += kBatch * rstep) {
-    uint4 c[kBatch];
+  for (int r = r0; r < nr; r += kStageBatch * rstep) {
+    uint4 c[kStageBatch];
 #pragma unroll
-    for (int q = 0; q < kBatch; ++q)
+    for (int q = 0; q < kStageBatch; ++q)
       c[q] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(src, vo + q * vstep, 0, 0));
 #pragma unroll
-    for (int q = 0; q < kBatch; ++q)
-      if (r + q * rstep < nr) stage_chunk<kDup>(dst + q * dstep, cq, c[q]);
-    vo += kBatch * vstep;
-    dst += kBatch * dstep;
+    for (int q = 0; q < kStageBatch; ++q)
+      if (r + q * rstep < nr) stage_chunk<true>(dst + q * dstep, cq, c[q]);
+    vo += kStageBatch * vstep;
+    dst += kStageBatch * dstep;
   }
 }
 
@@ -489,9 +486,9 @@ __global__ __launch_bounds__(long_threads(dup_cb(CB))) __attribute__((amdgpu_wav
   const int np = cb * kWaves + wave;
   const bool active = np < n_np;  // (halves form) idle waves still stage rows and meet the barriers
   constexpr bool kDup = dup_cb(CB);
-  const int part = long_part_steps(k_tiles, kDup), n_parts = ss / part;
+  const int part = long_part_steps(k_tiles), n_parts = ss / part;
   const int part_k = kStepTiles * part * 16;
-  const int xs_stride = long_row_words(k_tiles, kDup);
+  const int xs_stride = long_row_words(k_tiles);
   // plain rows: the double buffers are static, the dynamic LDS holds the slots only
   uint32_t *xs = smem;
   u32x4 *slot = reinterpret_cast<u32x4 *>(smem + (kDup ? kLongRows * xs_stride : 0)) + wave * slot_chunks(K);
@@ -515,7 +512,7 @@ __global__ __launch_bounds__(long_threads(dup_cb(CB))) __attribute__((amdgpu_wav
       for (int sl = 0; sl < n_sl; ++sl) {
         for (int pt = 0; pt < n_parts; ++pt) {
           const int k0 = (sl * n_parts + pt) * part_k;
-          stage_part<kDup, kStageBatchGu>(src, row_bytes, 2u * k0, q_row, q_lg, nr, xs, xs_stride);
+          stage_part(src, row_bytes, 2u * k0, q_row, q_lg, nr, xs, xs_stride);
           __syncthreads();
           if (active)
             qmv_slice_rb<K, CB, PD, NRB>(base, k_tiles, out / 16, k0 / 16, np, part, xs, xs_stride, nr, slot,
@@ -567,9 +564,9 @@ __global__ __launch_bounds__(long_threads(dup_cb(CB))) __attribute__((amdgpu_wav
   const int np = cb * kWaves + wave;
   const bool active = np < n_np;
   constexpr bool kDup = dup_cb(CB);
-  const int part = long_part_steps(k_tiles, kDup), n_parts = ss / part;
+  const int part = long_part_steps(k_tiles), n_parts = ss / part;
   const int part_k = kStepTiles * part * 16;
-  const int xs_stride = long_row_words(k_tiles, kDup);
+  const int xs_stride = long_row_words(k_tiles);
   const int q_row = part_k / 8;  // 16-byte chunks of act per row and part (a power of two)
   const int q_lg = __builtin_ctz(q_row);
   // plain rows: the double buffers are static, the dynamic LDS holds the slots only
@@ -591,7 +588,7 @@ __global__ __launch_bounds__(long_threads(dup_cb(CB))) __attribute__((amdgpu_wav
       for (int sl = 0; sl < n_sl; ++sl) {
         for (int pt = 0; pt < n_parts; ++pt) {
           const int k0 = (sl * n_parts + pt) * part_k;
-          stage_part<kDup, kStageBatchDn>(src, row_bytes, 2u * k0, q_row, q_lg, nr, xs, xs_stride);
+          stage_part(src, row_bytes, 2u * k0, q_row, q_lg, nr, xs, xs_stride);
           __syncthreads();
           if (active)
             qmv_slice_rb<K, CB, PD, NRB>(tb.tr[2], k_tiles, a.H / 16, k0 / 16, np, part, xs, xs_stride, nr,
@@ -634,7 +631,7 @@ static size_t expert_lds(int in, int pass_rows, int waves, int K, int cb) {
 // Long-run kernels: the staged rows (halves form; the plain form's double buffers are
 // static LDS), then one ring-word slot per wave.
 static size_t long_lds(int in, int K, int cb) {
-  return (dup_cb(cb) ? (size_t)kLongRows * long_row_words(in / 16, true) * 4 : 0) +
+  return (dup_cb(cb) ? (size_t)kLongRows * long_row_words(in / 16) * 4 : 0) +
          (size_t)(long_threads(dup_cb(cb)) / 64) * slot_chunks(K) * 16;
 }
 

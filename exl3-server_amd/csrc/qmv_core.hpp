@@ -96,14 +96,13 @@ __host__ __device__ constexpr int slice_words(int k_tiles, bool dup) {
 __host__ __device__ constexpr int staged_row_words(int k_tiles, bool dup) {
   return slice_words(k_tiles, dup) + 4;
 }
-// The long-run kernels stage a slice of duplicated rows in parts of at most 4 wave
-// steps (a part of 64 rows is ~66 KB of LDS, so that two 8-wave workgroups share a CU;
-// a whole slice of plain rows is that size already).
-__host__ __device__ constexpr int long_part_steps(int k_tiles, bool dup) {
-  return !dup || slice_steps(k_tiles) < 4 ? slice_steps(k_tiles) : 4;
+// The halves-form long-run kernels stage a slice of duplicated rows in parts of at most 4
+// wave steps (a part of 64 rows is ~66 KB of LDS, so that two 8-wave workgroups share a CU).
+__host__ __device__ constexpr int long_part_steps(int k_tiles) {
+  return slice_steps(k_tiles) < 4 ? slice_steps(k_tiles) : 4;
 }
-__host__ __device__ constexpr int long_row_words(int k_tiles, bool dup) {
-  return kStepTiles * long_part_steps(k_tiles, dup) * tile_words(dup) + 4;
+__host__ __device__ constexpr int long_row_words(int k_tiles) {
+  return kStepTiles * long_part_steps(k_tiles) * tile_words(true) + 4;
 }
 // 16-byte ring-word chunks of one wave's LDS slot: one wave step's 16K chunks, and at
 // least one per lane (every lane stores its first chunk register, K < 4 included).
@@ -426,41 +425,23 @@ __device__ __forceinline__ void mfma_quad_rb(const uint32_t (&W)[K + 1], const u
   }
 }
 
-// Long runs: RB blocks of 16 token rows share one decode. The B operands of a wave step
+// Halves form, long runs: RB blocks of 16 token rows share one decode. The B operands of a wave step
 // are decoded once and each block b runs the step's MFMAs with its own A operands
 // (staged row 16b + l%16 at word offset xo[b] of xs) and accumulators; per block a
 // step's MFMAs are exactly mfma_step's (the same operands in the same order).
 template <int K, int CB, int RB>
 __device__ __forceinline__ void mfma_step_rb(const uint32_t (&W)[K + 1], const uint32_t *xs,
                                              const int (&xo)[RB], f32x4 (&D)[RB][2]) {
+  static_assert(dup_cb(CB), "the reference form's long runs have their own step (moe_experts.hpp)");
   uint32_t F[K + 1];
   lane_funnels<K>(W, F);
-  if constexpr (!dup_cb(CB)) {
-    // k-rows 0..7 of the step (A0) before 8..15 (A1), as in mfma_step; two B operands
-    // live at a time
-    const f16x8 B0 = b_packed<K, CB, 0>(W, F), B1 = b_packed<K, CB, 4>(W, F);
-#pragma unroll
-    for (int r = 0; r < RB; ++r) {
-      const f16x8 A0 = lds_a(xs + xo[r]);
-      D[r][0] = mfma16(A0, B0, D[r][0]);
-      D[r][1] = mfma16(A0, B1, D[r][1]);
-    }
-    const f16x8 B2 = b_packed<K, CB, 16>(W, F), B3 = b_packed<K, CB, 20>(W, F);
-#pragma unroll
-    for (int r = 0; r < RB; ++r) {
-      const f16x8 A1 = lds_a(xs + xo[r] + 4);
-      D[r][0] = mfma16(A1, B2, D[r][0]);
-      D[r][1] = mfma16(A1, B3, D[r][1]);
-    }
-  } else {
-    mfma_quad_rb<K, CB, RB, 0>(W, F, xs, xo, D);
-    mfma_quad_rb<K, CB, RB, 1>(W, F, xs, xo, D);
-    mfma_quad_rb<K, CB, RB, 2>(W, F, xs, xo, D);
-    mfma_quad_rb<K, CB, RB, 3>(W, F, xs, xo, D);
-  }
+  mfma_quad_rb<K, CB, RB, 0>(W, F, xs, xo, D);
+  mfma_quad_rb<K, CB, RB, 1>(W, F, xs, xo, D);
+  mfma_quad_rb<K, CB, RB, 2>(W, F, xs, xo, D);
+  mfma_quad_rb<K, CB, RB, 3>(W, F, xs, xo, D);
 }
 
-// qmv_slice over up to 16 * RB staged token rows: xs = the first staged row (row
+// (Halves form) qmv_slice over up to 16 * RB staged token rows: xs = the first staged row (row
 // stride xs_stride words), nrows = rows staged (>= 1); rows past nrows read the last
 // row and are never stored. D[b] = the slice partials of rows 16b .. 16b + 15, from
 // zero, or (zero = false) continuing the accumulation already in D: a slice run as
