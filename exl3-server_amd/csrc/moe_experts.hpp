@@ -454,12 +454,12 @@ __device__ __forceinline__ int long_item(int b, int per_unit, int shared_mode, c
   return x * q + min(x, r) + (b >> 3);
 }
 
-// Waves per SIMD: 4, that is 128 registers; 3 for the instances that need 130 to 138. 48 experts
-// of 4096 x 1024 at 200 rows: K1 3inst 155 us with 22 registers spilled, 137 without; mcg K2,
-// K3 and K8, 6 to 8 spilled, 136, 139 and 165 against 134, 139 and 163.
-constexpr int gu_long_waves(int K, int CB) {
-  return (K == 1 && CB == 0) || ((K == 2 || K == 3 || K == 8) && CB == 1) ? 3 : 4;
-}
+// Waves per SIMD: 4, that is 128 registers; 3 for two instances that need 133 and 138. Whole
+// calls, us, 4 waves with spills against 3: K1 3inst (22 registers spilled), 48 experts of 4096 x
+// 1024 at 200 rows 155, 137, of 1024 x 512 64, 58, 160 of 1920 x 896 at 300 rows 168, 171; K8
+// mcg (8), the same three 165, 163; 62, 62; 210, 194. The mcg K2 and K3 instances (8 and 6) stay
+// at 4: 136, 134; 58, 57; 169, 172.
+constexpr int gu_long_waves(int K, int CB) { return (K == 1 && CB == 0) || (K == 8 && CB == 1) ? 3 : 4; }
 
 template <int K, int CB, int PD>
 __global__ __launch_bounds__(long_threads(dup_cb(CB))) __attribute__((amdgpu_waves_per_eu(gu_long_waves(K, CB), 8))) void k_moe_gate_up_long(MoeArgs a, int shared_mode, int dense_blocks) {

@@ -36,14 +36,15 @@ def kernels(path, tmp_path):
 
 
 @pytest.mark.skipif(not os.path.exists(READELF), reason="no llvm-readelf")
-@pytest.mark.parametrize("pattern,least", [
+@pytest.mark.parametrize("pattern,least,spilling", [
     # the linear of many rows: 8 widths x 3 codebooks x 3 tiles
-    (r"10k_qmv_rowsI", 72),
+    (r"10k_qmv_rowsI", 72, r"(?!)"),
     # the long-run expert kernels in the reference form, two steps in flight (the default): 2
-    # projections x 8 widths x 3 codebooks
-    (r"k_moe_(gate_up|down)_longILi\dELi[012]ELi2E", 48),
+    # projections x 8 widths x 3 codebooks; two instances are faster with 6 and 8 spilled
+    # registers than with a wave less
+    (r"k_moe_(gate_up|down)_longILi\dELi[012]ELi2E", 48, r"k_moe_gate_up_longILi[23]ELi1E"),
 ])
-def test_no_spills(pattern, least, tmp_path):
+def test_no_spills(pattern, least, spilling, tmp_path):
     found = {k: v for k, v in kernels(build.LIB_PATH, tmp_path).items() if re.search(pattern, k)}
     assert len(found) >= least
-    assert not {k: v for k, v in found.items() if v != (0, 0)}
+    assert not {k: v for k, v in found.items() if v[1] > (8 if re.search(spilling, k) else 0)}
