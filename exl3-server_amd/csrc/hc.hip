@@ -138,15 +138,15 @@ __device__ __forceinline__ void hc_chunk(const HcChunkRegs<NT, RT> &c, f32x4 (&E
       }
 }
 
-// Bound by the matrix unit and the stream reads together: 2048 positions of 4 x 4096 are 8.4 M
+// Bound by the matrix unit and the stream reads together: 2048 positions of 4 x 4096 are 1.05 M
 // 16x16x4 products (3/4 of their columns used; 13.7 us at 32 cycles each) over 67 MB (13 us at
 // the 5.1 TB/s of a copy). Measured there: 30.8 us, where a thread per projection, reading its
 // own row of the streams, took 474; two row tiles per wave, so that a loaded fn value serves 32
 // positions: 30.8 against 36 for one, and 33 for four (one wave per SIMD). At 4 positions both
 // forms are a round of loads: 4.6 us.
-// Workgroup (slice, RT row tiles, tiles of projections from NT * blockIdx.z): 4 waves of kC consecutive chunks each (kC = 1: the slice
-// is a group; kC = 4: a super-group), every chunk's loads issued one chunk ahead, then the
-// waves' sums added in order through LDS.
+// Workgroup (slice, RT row tiles, tiles of projections from NT * blockIdx.z): 4 waves of kC
+// consecutive chunks each (kC = 1: the slice is a group; kC = 4: a super-group), every chunk's
+// loads issued one chunk ahead, then the waves' sums added in order through LDS.
 template <int kN, int NT, int RT, int kC>
 __global__ __launch_bounds__(64 * kHcWaves) void k_hc_proj(const uint16_t *__restrict__ streams, int64_t P, int ND,
                                                            int W, const float *__restrict__ fn,
@@ -619,6 +619,8 @@ exl3_status check_hc(const exl3_hc_site *hc, int D) {
   return EXL3_OK;
 }
 
+// One partial per chunk: more than the groups' that calls of few positions write. Callers' sizes
+// (and which calls a given workspace is refused for) stay as they were with a partial per chunk.
 size_t hc_part_bytes(int N, int D, int64_t P) {
   return align_up((size_t)P * ((size_t)N * D / kHcChunk) * hc_vals(N) * 4, 256);
 }
@@ -667,8 +669,8 @@ exl3_status launch_hc_prepare(const exl3_hc_site *hc, const uint16_t *streams, i
                               float *comb, float *part, hipStream_t st) {
   if (P == 0) return EXL3_OK;
   const bool narrow = hc->mult <= kHcNarrowN;
-  // the positions of one call: bounded by the grid's second dimension (8 a workgroup, 3 with
-  // more than 4 streams)
+  // the positions of one call: 65,535 times 8, times 3 with more than 4 streams (a limit of the
+  // call; the launches' grids take more)
   const int rows = narrow ? 8 : 3;
   if ((P + rows - 1) / rows > 65535) return fail(EXL3_ERR_UNSUPPORTED, "too many positions in one call");
   if (narrow)

@@ -1061,8 +1061,9 @@ struct MoeLayout {
 
 // Calls of at least this many token rows take the long-run expert kernels (one
 // accumulator chain over the whole k range: within the reference's staged-path bound of
-// the short-run path, not bit-identical to it): EXL3_MOE_LONG_ROWS, read once, default 65
-// (at 64 rows the slice-parallel short-run kernels are still faster).
+// the short-run path, not bit-identical to it): EXL3_MOE_LONG_ROWS, read once, default 65. The
+// GLM-5 layer, spread routing, short against long: 64 rows 457, 465 us; 65 456, 466; 96 521,
+// 507; 128 564, 542; 256 663, 590; with 8 hot experts 64 rows 414, 433; 96 506, 491.
 int64_t long_min_rows() {
   static const int64_t v = [] {
     const char *e = std::getenv("EXL3_MOE_LONG_ROWS");
@@ -1154,6 +1155,8 @@ MoeLayout moe_layout(const exl3_moe_layer_s *L, int64_t N) {
   m.act = take(2 * (size_t)slots * m.Imax);
   m.S_dn = std::max(moe_slices(I), SI > 0 ? moe_slices(SI) : 1);
   m.yhat_dn = take(4 * (size_t)slots * m.S_dn * H);
+  // (the f16 shared expert's partials, also where it is two products, which need 2 N H bytes of
+  // dsh_dn alone: a call's size, and so which calls the scratch array holds, is one formula)
   m.dsh_gu = take(dense ? 4 * (size_t)2 * N * SI * kDenseSlots : 0);
   m.dsh_act = take(dense ? 2 * (size_t)N * SI : 0);
   m.dsh_dn = take(dense ? 4 * (size_t)N * H * kDenseSlots : 0);

@@ -157,7 +157,8 @@ typedef struct {
 typedef struct {
   int64_t calls;
   double router_ms;     /* logits + top-k routing + expert-order dispatch */
-  double gate_up_ms;    /* (input rotation +) routed gate|up (+ f16 shared gate/up) */
+  double gate_up_ms;    /* (input rotation +) routed gate|up (+ f16 shared gate/up, or all of a
+                           long call's large f16 shared expert) */
   double down_ms;       /* routed SwiGLU + down (+ f16 shared SwiGLU and down) */
   double combine_ms;    /* (a trellis shared expert on the caller's stream +) combine */
   double total_ms;
